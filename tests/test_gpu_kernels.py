@@ -337,6 +337,23 @@ def test_gemm_f32_with_few_rows_gives_the_bits_of_the_kernel_for_many(n, k):
         assert torch.equal(aligned, many[:2])
 
 
+@pytest.mark.parametrize("m, n, k", [(17, 33, 4), (33, 2050, 68), (64, 31, 64), (65, 8200, 96), (300, 6161, 100), (130, 16500, 36),
+                                     (1030, 16500, 60), (2048, 16384, 32)])
+@pytest.mark.parametrize("aligned", [True, False])
+def test_gemm_f32_tiles_give_the_bits_of_the_kernel_for_few_rows(m, n, k, aligned):
+    """Small, middle and large tiles (chosen by rows and columns), whole and cut off at every edge, K no multiple of a step
+    or of a group of 16, rows on 16-byte boundaries and not: every element is the same chain of sums as in a step of few
+    rows, and within (k / 16 + 16) roundings of the 64-bit product of the magnitudes."""
+    torch.manual_seed(m + n + k)
+    x = torch.randn(m, k + (0 if aligned else 1), device=DEV)[:, :k]
+    w = torch.randn(n, k + (0 if aligned else 3), device=DEV)[:, :k]
+    got = _ops().gemm_f32(x, w)
+    bound = (k / 16 + 16) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert bool(((got.double() - x.double() @ w.double().T).abs() <= bound).all())
+    for first in (0, max(m // 2 - 5, 0), m - 9):
+        assert torch.equal(_ops().gemm_f32(x[first : first + 9], w), got[first : first + 9])
+
+
 # ----------------------------------------------------------------------------- attention
 def _paged(k, v, page, n_pages, seed=0, dtype=torch.float32):
     """Scatter dense per-request keys/values [S, Hkv, dh] into shuffled pages; returns pages and

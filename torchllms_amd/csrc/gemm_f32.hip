@@ -1,145 +1,227 @@
-// C[M, N] = A[M, K] * W[N, K]^T in true 32-bit: float inputs, float FMA accumulation, no matrix-core
-// reduced-precision mode.  Each output element is accumulated by one thread over k = 0..K-1 in
-// ascending order (in groups of 16 that are added up first), so its value does not depend on M or on
-// where the row sits in the batch.
-// Throughput is secondary: this is the matrix product of the 32-bit path.
-#include <type_traits>
-
+// C[M, N] = A[M, K] * W[N, K]^T in true 32-bit: float inputs, every product and sum rounded to float, no
+// reduced-precision mode.  An output element is the sum over groups of 16 products: a group's products are chained by
+// fused multiply-adds from k ascending, starting from zero, and its sum joins the running sum, groups in ascending order.
+// (The rounding error of a long sum grows with the number of additions to one accumulator: this way there are K / 16 + 16
+// of them instead of K.)  So a value depends neither on M nor on where the row sits in the batch, whichever kernel
+// computes it: tiles on the matrix cores for prompts, a wave per four columns for up to 16 rows.
 #include "common.h"
+#include "recurrence.h"  // mfma_f32
 
 namespace {
 
 constexpr int BK = 16;  // products that are added among themselves before they join the running sum
 
-// A block computes a BM x BN tile of C with (BM / TM) x (BN / TN) = 256 threads, each a TM x TN piece of it
-// (its rows and columns in runs of four, so that operands come from LDS sixteen bytes at a time).  Tiles of A
-// and W, BK wide, pass through LDS transposed (k-major); the next tiles travel from memory into registers
-// while the current ones are multiplied, and two sets of LDS tiles leave one barrier a step.
-// Two shapes: 64 x 64 with 4 x 4 a thread for steps of a few dozen rows, 128 x 128 with 8 x 8 a thread for
-// prompts (twice the arithmetic per byte read from LDS).  The arithmetic of an output element is the same in
-// both, and in the kernel for few rows below: the BK products of a step chained by fused multiply-adds from k
-// ascending, starting from zero, then added to the running sum.
-template <int BM, int BN, int TM, int TN>
-__global__ void __launch_bounds__((BM / TM) * (BN / TN))
-gemm_f32_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
-                float* __restrict__ C, int ldc, int M, int N, int K) {
-  constexpr int kThreads = (BM / TM) * (BN / TN);
-  static_assert(kThreads == 256 && TM % 4 == 0 && TN % 4 == 0, "256 threads, pieces in runs of four");
-  constexpr int kPerA = BM * BK / kThreads;  // elements of a tile that one thread moves: a run along k
-  constexpr int kPerW = BN * BK / kThreads;
-  static_assert(kPerA % 4 == 0 && kPerW % 4 == 0 && BK % kPerA == 0 && BK % kPerW == 0, "runs of whole float4s");
-  constexpr int kPitchA = BM + 4, kPitchW = BN + 4;
-  constexpr int kAhead = TM * TN >= 64 ? 2 : 4;  // steps of k whose operands are in registers together
-  __shared__ __attribute__((aligned(16))) float As[2][BK][kPitchA];
-  __shared__ __attribute__((aligned(16))) float Ws[2][BK][kPitchW];
+// ----------------------------------------------------------------------------- prompts
+// v_mfma_f32_16x16x4_f32 computes an element as four fused multiply-adds chained from depth 0 up, each rounded to float
+// (checked against fmaf bit for bit over a million groups of 16, values of 2^-30 to 2^30 and denormal ones): four of them
+// from a zero accumulator are a group.  It does 143 to 155 TFLOP/s here where fused multiply-adds issued from registers
+// reach 113, needs a fraction of the LDS reads, and a few chains a wave keep a SIMD busy.  What bounds it: the running sums'
+// additions and the LDS reads take turns with the MFMAs (an addition an MFMA alone: 127 of 143 with two waves a SIMD).
+//   * a block of four waves takes a BM x BN tile of C, a wave a WM x WN piece of it; K is walked in steps of 32 or 64;
+//   * the step's rows of A and W lie in LDS as they are in memory, 128 or 256 bytes a row; 16-byte piece p of row r at slot
+//     p ^ (r / 2 % 8) or p ^ (r % 16), so that the 16 rows x 4 words that a wave's operand read takes fall on all 64 banks;
+//   * with 16-byte rows (kVec) the pieces go straight to LDS (global_load_lds), kStages - 1 steps ahead; otherwise they
+//     pass through registers element by element, one step ahead;
+//   * rows past M and N repeat the last row (their results are not stored), elements past K are zeros: a chain that goes
+//     on with zeros keeps its bits.
+// C^T tiles (W the first operand): a lane holds four neighbouring columns of a row of C.
+// 562 rows of the 1B shape's qkv, o, gate/up and down matrices: 434 us on average for all but gate/up and 758 for that with
+// tiles of plain fused multiply-adds before, 95 + 73 + 388 + 266 now; 2,048 rows of the 8B shape's gate/up: 4.0 ms, 120 TFLOP/s.
+__device__ __attribute__((aligned(16))) const float kZeroPiece[4] = {0.f, 0.f, 0.f, 0.f};
+
+// 64 lanes x 16 bytes from `src` (per lane) to LDS at byte offset `lds_at` (wave-uniform) + 16 * lane.  Assembly for the
+// reason gemm_wide.hip gives: the kernel counts its loads itself.
+__device__ __forceinline__ void piece_to_lds(const float* src, uint32_t lds_at) {
+  asm volatile(
+      "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %0, off"
+      :
+      : "v"(src), "s"(lds_at)
+      : "m0", "memory");
+}
+
+template <int BM, int BN, int WM, int WN, int kStepF, int kStages, bool kVec>
+__global__ void __launch_bounds__(256, 2)  // (two waves a SIMD: with 256 registers the compiler keeps sums out of the accumulation registers)
+gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw, float* __restrict__ C, int ldc, int M,
+                     int N, int K) {
+  static_assert((BM / WM) * (BN / WN) == 4, "four waves");
+  constexpr int MT = WM / 16, NT = WN / 16;
+  constexpr int kRowPieces = kStepF / 4;
+  constexpr int kTurn = 64 / kStepF;             // rows that lie on the 64 banks side by side
+  constexpr int kStage = (BM + BN) * kStepF;     // floats of one buffer: rows of A, then rows of W
+  constexpr int kLoads = (BM + BN) * kRowPieces / 256;  // load instructions of a wave per step: a KB each
+  constexpr int kPending = (kStages - 2) * kLoads;
+  static_assert(kPending < 64, "vmcnt has six bits");
+  // s_waitcnt that leaves the loads of the kStages - 2 latest steps outstanding
+  constexpr int kWaitOldest = (kPending & 0xF) | (0x7 << 4) | (0xF << 8) | ((kPending >> 4) << 14);
+  extern __shared__ __attribute__((aligned(16))) float tiles[];
   const int tid = threadIdx.x;
-  const int tx = tid % (BN / TN);  // column group
-  const int ty = tid / (BN / TN);  // row group
+  const int wave = tid / kWave, lane = tid % kWave;
+  const int n16 = lane % 16, g4 = lane / 16;
   // consecutive blocks share their columns: the tile of W is read from memory once for all of them
-  const int m0 = blockIdx.x * BM;
-  const int n0 = blockIdx.y * BN;
-  // run r of the thread's rows is rows (BM / (TM / 4)) * r + 4 * ty ... + 3 of the tile; columns likewise
-  constexpr int kRowRun = BM / (TM / 4), kColRun = BN / (TN / 4);
+  const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
+  const int wm = (wave % (BM / WM)) * WM, wn = (wave / (BM / WM)) * WN;
+  const int steps = (K + kStepF - 1) / kStepF;
 
-  float acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = 0.f;
+  // row r of a buffer: row of A, or of W behind them; a clamped row of memory
+  auto row_of = [&](int r) { return r < BM ? A + (size_t)min(m0 + r, M - 1) * lda : W + (size_t)min(n0 + r - BM, N - 1) * ldw; };
 
-  // what this thread moves: row (of A or of W) and the run of k within the step
-  const int ar = tid / (BK / kPerA), ak = (tid % (BK / kPerA)) * kPerA;
-  const int wr = tid / (BK / kPerW), wk = (tid % (BK / kPerW)) * kPerW;
-  const bool a_vec = (lda % 4) == 0 && ((uintptr_t)A % 16) == 0;
-  const bool w_vec = (ldw % 4) == 0 && ((uintptr_t)W % 16) == 0;
-  const float* a_row = A + (size_t)min(m0 + ar, M - 1) * lda;
-  const float* w_row = W + (size_t)min(n0 + wr, N - 1) * ldw;
-  const bool a_in = m0 + ar < M, w_in = n0 + wr < N;
-  float ra[kPerA], rw[kPerW];
-  auto fetch_run = [&](const float* row, bool inside, bool vec, int k, float* dst, auto per) {
-    constexpr int kPer = decltype(per)::value;
-    if (inside && vec && k + kPer <= K) {
+  // -- aligned rows: instruction j of the wave fills buffer rows 8 (wave kLoads + j) ... + 7, a lane one slot of one row
+  const float* src[kLoads];
+  const uint32_t lds_base = (uint32_t)(uintptr_t)tiles;
+  const uint32_t at0 = __builtin_amdgcn_readfirstlane(lds_base + wave * kLoads * 1024);
+  int piece[kLoads];
+  if constexpr (kVec) {
 #pragma unroll
-      for (int u = 0; u < kPer; u += 4) {
-        const float4 v = *reinterpret_cast<const float4*>(row + k + u);
-        dst[u] = v.x; dst[u + 1] = v.y; dst[u + 2] = v.z; dst[u + 3] = v.w;
+    for (int j = 0; j < kLoads; ++j) {
+      const int r = (64 / kRowPieces) * (wave * kLoads + j) + lane / kRowPieces;
+      piece[j] = 4 * ((lane % kRowPieces) ^ (r / kTurn % kRowPieces));
+      src[j] = row_of(r);
+    }
+  }
+  auto issue = [&](int step, int buffer) {
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) {
+      const int k = step * kStepF + piece[j];
+      piece_to_lds(k < K ? src[j] + k : kZeroPiece, at0 + buffer * kStage * (int)sizeof(float) + j * 1024);
+    }
+  };
+  // -- other rows: a thread moves pieces tid, tid + 256, ... of the buffer
+  constexpr int kMoves = (BM + BN) * kRowPieces / 256;
+  float held[kMoves][4];
+  auto fetch = [&](int step) {
+#pragma unroll
+    for (int j = 0; j < kMoves; ++j) {
+      const int r = (tid + 256 * j) / kRowPieces, k = step * kStepF + 4 * (tid % kRowPieces);
+      const float* row = row_of(r);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) held[j][e] = k + e < K ? row[k + e] : 0.f;
+    }
+  };
+  auto put = [&](int buffer) {
+#pragma unroll
+    for (int j = 0; j < kMoves; ++j) {
+      const int r = (tid + 256 * j) / kRowPieces;
+      *reinterpret_cast<float4*>(tiles + buffer * kStage + r * kStepF + 4 * ((tid % kRowPieces) ^ (r / kTurn % kRowPieces))) =
+          float4{held[j][0], held[j][1], held[j][2], held[j][3]};
+    }
+  };
+
+  f32x4_t acc[NT][MT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int c = 0; c < MT; ++c) acc[t][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  // word offsets of the lane's operands within 16 rows: piece p of row n16, depth g4 of its four
+  int word[kRowPieces];
+#pragma unroll
+  for (int p = 0; p < kRowPieces; ++p) word[p] = n16 * kStepF + 4 * (p ^ (n16 / kTurn % kRowPieces)) + g4;
+  auto multiply = [&](int buffer) {
+    const float* as = tiles + buffer * kStage + wm * kStepF;
+    const float* ws = tiles + buffer * kStage + (BM + wn) * kStepF;
+constexpr int kGroups = kStepF / BK;
+    if constexpr (MT * NT == 1) {
+      // one tile: the step's groups are the chains that run side by side
+      float w[kRowPieces], a[kRowPieces];
+#pragma unroll
+      for (int p = 0; p < kRowPieces; ++p) {
+        w[p] = ws[word[p]];
+        a[p] = as[word[p]];
       }
+      f32x4_t part[kGroups];
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int g = 0; g < kGroups; ++g) part[g] = mfma_f32(w[4 * g + s], a[4 * g + s], s == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : part[g]);
+#pragma unroll
+      for (int g = 0; g < kGroups; ++g)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[0][0][i] += part[g][i];
     } else {
+      // a row of MT tiles at a time: its chains run side by side, and between its MFMAs stand the additions of the row
+      // before it, so that the matrix core does not wait for them; operands of the next group are read during this one
+      float w[2][4][NT], a[2][4][MT];
+      auto operands = [&](int g) {
 #pragma unroll
-      for (int u = 0; u < kPer; ++u) dst[u] = (inside && k + u < K) ? row[k + u] : 0.f;
+        for (int s = 0; s < 4; ++s) {
+#pragma unroll
+          for (int t = 0; t < NT; ++t) w[g & 1][s][t] = ws[t * 16 * kStepF + word[4 * g + s]];
+#pragma unroll
+          for (int c = 0; c < MT; ++c) a[g & 1][s][c] = as[c * 16 * kStepF + word[4 * g + s]];
+        }
+      };
+      f32x4_t part[2][MT];
+      operands(0);
+#pragma unroll
+      for (int u = 0; u <= kGroups * NT; ++u) {
+        const int g = u / NT, t = u % NT;
+        if (t == 0 && g + 1 < kGroups) operands(g + 1);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          // (the order as written: left to itself the compiler starts all rows at once and spills)
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int c = 0; c < MT; ++c) {
+            if (u < kGroups * NT) part[u & 1][c] = mfma_f32(w[g & 1][s][t], a[g & 1][s][c], s == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : part[u & 1][c]);
+            if (u > 0) acc[(u - 1) % NT][c][s] += part[(u - 1) & 1][c][s];
+          }
+        }
+      }
     }
-  };
-  auto fetch = [&](int k0) {
-    fetch_run(a_row, a_in, a_vec, k0 + ak, ra, std::integral_constant<int, kPerA>{});
-    fetch_run(w_row, w_in, w_vec, k0 + wk, rw, std::integral_constant<int, kPerW>{});
-  };
-  auto store = [&](int buffer) {
-#pragma unroll
-    for (int u = 0; u < kPerA; ++u) As[buffer][ak + u][ar] = ra[u];
-#pragma unroll
-    for (int u = 0; u < kPerW; ++u) Ws[buffer][wk + u][wr] = rw[u];
   };
 
-  fetch(0);
-  store(0);
-  __syncthreads();
-  int buffer = 0;
-  for (int k0 = 0; k0 < K; k0 += BK) {
-    const bool more = k0 + BK < K;
-    if (more) fetch(k0 + BK);
-    // the BK products of this step are added among themselves first and then to the running sum:
-    // the rounding error of a long sum grows with the number of additions to one accumulator, and
-    // this way there are K / BK + BK of them instead of K (at K = 1024 the 32-bit model's distance
-    // from a 64-bit computation halves); the order is still fixed by K alone
-    float part[TM][TN];
+  if constexpr (kVec) {
+    // all loads are unconditional (past the end the last step is fetched again and never used), so that a wave's count of
+    // outstanding loads is the same in every trip
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) part[i][j] = 0.f;
-    // (unrolled by kAhead only: unrolled whole, the compiler asks for all sixteen steps' operands at once
-    // and the large tile takes 405 registers)
-#pragma unroll kAhead
-    for (int k = 0; k < BK; ++k) {
-      float a[TM], w[TN];
-#pragma unroll
-      for (int r = 0; r < TM / 4; ++r) {
-        const float4 v = *reinterpret_cast<const float4*>(&As[buffer][k][kRowRun * r + 4 * ty]);
-        a[4 * r] = v.x; a[4 * r + 1] = v.y; a[4 * r + 2] = v.z; a[4 * r + 3] = v.w;
-      }
-#pragma unroll
-      for (int r = 0; r < TN / 4; ++r) {
-        const float4 v = *reinterpret_cast<const float4*>(&Ws[buffer][k][kColRun * r + 4 * tx]);
-        w[4 * r] = v.x; w[4 * r + 1] = v.y; w[4 * r + 2] = v.z; w[4 * r + 3] = v.w;
-      }
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) part[i][j] = fmaf(a[i], w[j], part[i][j]);
+    for (int s = 0; s < kStages - 1; ++s) issue(min(s, steps - 1), s);
+    int buffer = 0;
+    for (int i = 0; i < steps; ++i) {
+      // this wave's loads of step i have landed; after the barrier everybody's have, and everybody has finished with
+      // step i - 1, whose buffer the next loads overwrite
+      __builtin_amdgcn_s_waitcnt(kWaitOldest);
+      __syncthreads();
+      issue(min(i + kStages - 1, steps - 1), buffer == 0 ? kStages - 1 : buffer - 1);
+      multiply(buffer);
+      buffer = buffer + 1 == kStages ? 0 : buffer + 1;
     }
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] += part[i][j];
-    if (more) store(buffer ^ 1);
+    __builtin_amdgcn_s_waitcnt(0);  // the last, unused fetches must not land after the block has gone
+  } else {
+    fetch(0);
+    put(0);
     __syncthreads();
-    buffer ^= 1;
-  }
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int m = m0 + kRowRun * (i / 4) + 4 * ty + i % 4;
-    if (m >= M) continue;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int n = n0 + kColRun * (j / 4) + 4 * tx + j % 4;
-      if (n < N) C[(size_t)m * ldc + n] = acc[i][j];
+    for (int i = 0; i < steps; ++i) {
+      if (i + 1 < steps) fetch(i + 1);
+      multiply(i & 1);
+      if (i + 1 < steps) put((i + 1) & 1);
+      __syncthreads();
     }
   }
+
+  // acc[t][c][i] = C[m0 + wm + 16 c + n16][n0 + wn + 16 t + 4 g4 + i]
+  const bool whole = ldc % 4 == 0 && (uintptr_t)C % 16 == 0;
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int c = 0; c < MT; ++c) {
+      const int m = m0 + wm + 16 * c + n16, n = n0 + wn + 16 * t + 4 * g4;
+      if (m >= M) continue;
+      float* dst = C + (size_t)m * ldc + n;
+      if (whole && n + 4 <= N) {
+        *reinterpret_cast<f32x4_t*>(dst) = acc[t][c];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (n + i < N) dst[i] = acc[t][c][i];
+      }
+    }
 }
 
 // ----------------------------------------------------------------------------- few rows (decode steps)
-// The kernel above gives a block 64 rows of A; a decode step has one to sixteen, and its grid is then
-// N / 64 blocks that walk all of K in steps of 16 with two barriers each: a 4096 x 14336 matrix took
-// over a millisecond.  This kernel computes the very same arithmetic for every output element (groups
+// The kernel above gives a block 32 rows of A and more; a decode step has one to sixteen, and what counts is reading W
+// from everywhere at once.  This kernel computes the very same arithmetic for every output element (groups
 // of 16 products, chained by fused multiply-adds from k ascending, each group's sum added to the
 // running sum in the order of the groups), so its results are the same bits, but spreads the groups
 // of an element over the lanes of a wave:
@@ -296,6 +378,40 @@ gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __restri
   }
 }
 
+template <int BM, int WM, int kStepF, int kStages, bool kVec>
+int launch_tile(const float* A, int lda, const float* W, int ldw, float* C, int ldc, int M, int N, int K, hipStream_t stream) {
+  constexpr size_t kLds = (size_t)kStages * (2 * BM) * kStepF * sizeof(float);
+  const dim3 grid((M + BM - 1) / BM, (N + BM - 1) / BM);
+  TL_REQUIRE(grid.y <= 65535, "gemm_f32: N=%d exceeds the grid limit of one launch", N);
+  if (kLds > 48 * 1024) {
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_f32_tile_kernel<BM, BM, WM, WM, kStepF, kStages, kVec>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds);
+    if (e != hipSuccess) return tl_fail(TL_ERR_HIP, "gemm_f32: %s", hipGetErrorString(e));
+  }
+  gemm_f32_tile_kernel<BM, BM, WM, WM, kStepF, kStages, kVec><<<grid, 256, kLds, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+  return tl_check_launch("gemm_f32_tile");
+}
+
+// Which tile: 128 x 128, 64 x 64 or 32 x 32.  A launch takes as long as the fullest CU, so its time is about fixed + per x
+// (blocks of the fullest CU); with K = 2,048 measured 30 + 141 us for the large tile (16,384 columns of 2,048 rows: 1,160 us,
+// 118 TFLOP/s), 20 + 39 for the middle one (562 rows of them: 387 against 545 and 461 for the others) and 10 + 12 for the
+// small one (2,048 columns of 562 rows: 73 against 94 and 181).
+int launch_tiles(const float* A, int lda, const float* W, int ldw, float* C, int ldc, int M, int N, int K, hipStream_t stream) {
+  const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0;
+  const size_t cus = (size_t)tl_device_facts().compute_units;
+  auto cost = [&](int tile, double fixed, double per) {
+    const size_t blocks = (size_t)((M + tile - 1) / tile) * ((N + tile - 1) / tile);
+    return fixed + per * (double)((blocks + cus - 1) / cus);
+  };
+  const double large = cost(128, 30.0, 141.0), middle = cost(64, 20.0, 39.0), small = cost(32, 10.0, 12.1);
+  if (!vec)  // (the large tile's rows would not fit into registers on their way)
+    return middle <= small ? launch_tile<64, 32, 32, 2, false>(A, lda, W, ldw, C, ldc, M, N, K, stream)
+                           : launch_tile<32, 16, 64, 2, false>(A, lda, W, ldw, C, ldc, M, N, K, stream);
+  if (large <= middle && large <= small) return launch_tile<128, 64, 32, 2, true>(A, lda, W, ldw, C, ldc, M, N, K, stream);
+  if (middle <= small) return launch_tile<64, 32, 32, 3, true>(A, lda, W, ldw, C, ldc, M, N, K, stream);
+  return launch_tile<32, 16, 64, 3, true>(A, lda, W, ldw, C, ldc, M, N, K, stream);
+}
+
 }  // namespace
 
 TL_EXPORT int tl_gemm_f32(const float* A, int lda, const float* W, int ldw, float* C, int ldc, int M, int N,
@@ -330,15 +446,5 @@ TL_EXPORT int tl_gemm_f32(const float* A, int lda, const float* W, int ldw, floa
 #undef TL_ROWS_LAUNCH
     return tl_check_launch("gemm_f32_rows");
   }
-  // prompts take the large tile, if that still makes a block for every CU (both give the same sums)
-  if (M > 96 && (size_t)((M + 127) / 128) * ((N + 127) / 128) >= 256) {
-    const unsigned gy = (N + 127) / 128;
-    TL_REQUIRE(gy <= 65535, "gemm_f32: N=%d exceeds the grid limit of one launch", N);
-    gemm_f32_kernel<128, 128, 8, 8><<<dim3((M + 127) / 128, gy), 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
-  } else {
-    const unsigned gy = (N + 63) / 64;
-    TL_REQUIRE(gy <= 65535, "gemm_f32: N=%d exceeds the grid limit of one launch", N);
-    gemm_f32_kernel<64, 64, 4, 4><<<dim3((M + 63) / 64, gy), 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
-  }
-  return tl_check_launch("gemm_f32");
+  return launch_tiles(A, lda, W, ldw, C, ldc, M, N, K, stream);
 }
