@@ -3,6 +3,7 @@
 import math
 
 import pytest
+import numpy as np
 import torch
 import torch.nn.functional as F
 
@@ -352,6 +353,35 @@ def test_gemm_f32_tiles_give_the_bits_of_the_kernel_for_few_rows(m, n, k, aligne
     assert bool(((got.double() - x.double() @ w.double().T).abs() <= bound).all())
     for first in (0, max(m // 2 - 5, 0), m - 9):
         assert torch.equal(_ops().gemm_f32(x[first : first + 9], w), got[first : first + 9])
+
+
+# ----------------------------------------------------------------------------- routed experts' products by tiles
+@pytest.mark.parametrize("counts, D, F", [
+    ([1], 64, 64), ([0, 3, 0, 17, 1, 0], 128, 192), ([15, 16, 17, 33], 64, 320), ([31, 0, 32, 65], 192, 64), ([64, 63, 129, 0, 65], 128, 448),
+    ([127, 128, 129], 64, 192), ([300, 1, 0, 520], 320, 128), ([513], 64, 64), ([2, 0, 1] * 30, 64, 128), ([0, 0, 40] * 44, 64, 64)])
+def test_expert_products_by_tiles(counts, D, F):
+    """Every tile size (chosen by the mean rows of an expert), experts without rows, one row, a tile's edge, columns that
+    are no multiple of a tile, one step along K, more experts than a wave has lanes, and rows behind the last expert's
+    (pairs of outputs that are no experts), which stay unwritten."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(sum(counts) + D)
+    E, rest = len(counts), 5
+    rows = torch.randn(sum(counts) + rest, D, generator=g).bfloat16()
+    gu, down = ((torch.randn(E, *s, generator=g) * 0.1).bfloat16() for s in ((2 * F, D), (D, F)))
+    offsets = torch.tensor([0] + list(np.cumsum(counts)) + [sum(counts) + rest], dtype=torch.int32)
+    mid = ops.expert_glu_rows(rows.to(DEV), gu.to(DEV), offsets.to(DEV)).cpu()
+    y = ops.expert_down_rows(mid.to(DEV), down.to(DEV), offsets.to(DEV)).cpu()
+    for e in range(E):
+        at = slice(int(offsets[e]), int(offsets[e + 1]))
+        x, w = rows[at].double(), gu[e].double()
+        gate, up = x @ w[:F].T, x @ w[F:].T
+        # 32-bit sums of exact products (K roundings of the magnitudes at most), |silu'| <= 1.1, one rounding to bfloat16
+        slack = D * 2.0 ** -24 * (x.abs() @ w.abs().T)
+        want = torch.nn.functional.silu(gate) * up
+        bound = 2.0 ** -8 * want.abs() + 1.2 * (slack[:, :F] * up.abs() + slack[:, F:] * (gate.abs() + 1.0)) + 1e-6
+        assert bool(((mid[at].double() - want).abs() <= bound).all())
+        x, w = mid[at].double(), down[e].double()
+        assert bool(((y[at].double() - x @ w.T).abs() <= F * 2.0 ** -24 * (x.abs() @ w.abs().T) + 1e-30).all())
 
 
 # ----------------------------------------------------------------------------- attention

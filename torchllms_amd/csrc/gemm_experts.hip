@@ -1,0 +1,257 @@
+// The products of routed experts over their gathered rows, bfloat16 inputs, 32-bit sums: for every expert e,
+// C[r, n] = rows[r] . W[e][n] for its rows offsets[e] .. offsets[e + 1], or (GLU) mid[r, n] = silu(rows[r] . Wgate[e][n]) *
+// (rows[r] . Wup[e][n]), rounded once.  How many rows an expert got is known on the device only, so one launch covers all
+// experts: a block finds its tile from the offsets, and blocks beyond the last tile end at once.  Nothing is read back, and
+// the launch depends on the step's shape alone (it can be recorded).
+//
+//   * A block of four waves takes BM rows of one expert and BN rows of its matrix; K is walked in steps of 64.  A step's
+//     rows lie in LDS as in memory, 128 bytes a row, 16-byte piece p of row r at slot p ^ (r % 8): the eight lanes that are
+//     served together read eight different slots.  Everything is fetched by global_load_lds, kStages - 1 steps ahead.
+//   * C^T by MFMA 16x16x32 (first operand W): a lane holds four neighbouring columns of a row.  Operands of one half of a
+//     step are read while the other half is multiplied; the one barrier a step stands between the two halves, so that
+//     neither the wait for LDS nor that for the barrier leaves the matrix cores idle.
+//   * GLU: a wave's rows of W are half gate rows, half up rows of the same columns, so the gate meets its up product in
+//     registers.
+//   * Tiles by the rows an expert has on average: 128 x 128 for prompts (bound by LDS reads and the matrix cores, which take
+//     about the same time; two blocks a CU fill each other's gaps), 16, 32 or 64 rows for decode steps and short prompts
+//     (bound by reading W: many blocks with several steps in flight).
+//   * Blocks go to the eight XCDs in turn.  All row tiles of one (expert, column tile) go to the same XCD one after the
+//     other, so W is read from memory once and met again in that XCD's L2; an expert's column tiles are spread over all XCDs.
+// 8 experts of 4,096 x 3,584, gated + plain product: 16 pairs 119 us (a wave per 16 columns with operands straight from memory,
+// before: 156; the bytes of W at 6.1 TB/s: 101), 128 pairs 134 (235; 116), 4,096 pairs 518 (a library product per expert, with
+// the activation in a kernel of its own: 632, and the host waited for the offsets once a layer) = 697 TFLOP/s.
+#include "common.h"
+
+namespace {
+
+typedef __bf16 bf16x8_e __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4_e __attribute__((ext_vector_type(4)));
+typedef float float4_e __attribute__((ext_vector_type(4)));
+
+constexpr int kStepE = 64;    // k per step: 8 pieces of 16 bytes a row
+constexpr int kXcds = 8;
+
+// 64 lanes x 16 bytes from `src` (per lane) to LDS at byte offset `lds_at` (wave-uniform) + 16 * lane; assembly because the
+// kernel counts its loads itself (see gemm_wide.hip).
+__device__ __forceinline__ void rows_to_lds(const bf16_t* src, uint32_t lds_at) {
+  asm volatile(
+      "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %0, off"
+      :
+      : "v"(src), "s"(lds_at)
+      : "m0", "memory");
+}
+
+template <int BM, int BN, int WAVES_M, int kStages, bool GLU>
+struct ExpertTile {
+  static constexpr int kWavesN = 4 / WAVES_M;
+  static constexpr int WM = BM / WAVES_M, WN = BN / kWavesN;
+  static constexpr int MT = WM / 16, NT = WN / 16;
+  static constexpr int kColumns = GLU ? BN / 2 : BN;           // output columns of a block
+  static constexpr int kALoads = BM >= 32 ? BM / 32 : 1;       // load instructions of a wave per step: 8 rows each
+  static constexpr int kWLoads = BN / 32;
+  static constexpr int kStage = (BM + BN) * kStepE;            // elements of one buffer
+  static constexpr int kLdsBytes = kStages * kStage * 2;
+  static constexpr int kPending = (kStages - 2) * (kALoads + kWLoads);
+  static_assert(kPending < 64, "vmcnt has six bits");
+  // s_waitcnt that leaves the loads of the kStages - 2 latest steps outstanding
+  static constexpr int kWait = (kPending & 0xF) | (0x7 << 4) | (0xF << 8) | ((kPending >> 4) << 14);
+};
+
+template <int BM, int BN, int WAVES_M, int kStages, bool GLU>
+__global__ void __launch_bounds__(256)
+expert_tile_kernel(const bf16_t* __restrict__ rows, const bf16_t* __restrict__ w, const int32_t* __restrict__ offsets, int n_experts,
+                   bf16_t* __restrict__ mid, float* __restrict__ y, int K, int N) {
+  using S = ExpertTile<BM, BN, WAVES_M, kStages, GLU>;
+  constexpr int MT = S::MT, NT = S::NT;
+  extern __shared__ __attribute__((aligned(16))) bf16_t lds_e[];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int n16 = lane % 16, g4 = lane / 16;
+
+  // which tile: XCD x walks, expert after expert, its column tiles n = x, x + 8, ... (the start shifted from expert to
+  // expert, so that a number of tiles that is no multiple of 8 evens out), the row tiles of each side by side
+  const int n_tiles = (N + S::kColumns - 1) / S::kColumns;
+  const int per_xcd = (n_tiles + kXcds - 1) / kXcds;
+  const int x = blockIdx.x % kXcds;
+  int j = blockIdx.x / kXcds;  // place among this XCD's tiles
+  int e = -1, m_tiles = 0;
+  for (int e0 = 0; e0 < n_experts; e0 += kWave) {
+    const int mine = e0 + lane < n_experts ? (offsets[e0 + lane + 1] - offsets[e0 + lane] + BM - 1) / BM : 0;
+    int sum = mine;  // row tiles up to and with this expert
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const int before = __shfl_up(sum, off, kWave);
+      if (lane >= off) sum += before;
+    }
+    const unsigned long long beyond = __ballot(sum * per_xcd > j);
+    if (beyond) {
+      const int l = __ffsll(beyond) - 1;
+      e = e0 + l;
+      m_tiles = __shfl(mine, l, kWave);
+      j -= (__shfl(sum, l, kWave) - m_tiles) * per_xcd;
+      break;
+    }
+    j -= __shfl(sum, kWave - 1, kWave) * per_xcd;
+  }
+  if (e < 0) return;
+  e = __builtin_amdgcn_readfirstlane(e);
+  const int n_tile = __builtin_amdgcn_readfirstlane((j / m_tiles) * kXcds + (x + e * (n_tiles % kXcds)) % kXcds);
+  if (n_tile >= n_tiles) return;
+  const int hi = offsets[e + 1];
+  const int r0 = __builtin_amdgcn_readfirstlane(offsets[e] + (j % m_tiles) * BM);
+  const int n0 = n_tile * S::kColumns;
+  const bf16_t* we = w + (size_t)e * (GLU ? 2 : 1) * N * K;
+
+  // what this lane fetches: rows past the expert's last repeat it, columns past N likewise; neither result is stored
+  const int q8 = lane / 8, piece = 8 * ((lane % 8) ^ q8);
+  const bf16_t* asrc[S::kALoads];
+  const int a_first = BM >= 32 ? wave * S::kALoads * 8 : (wave % (BM / 8)) * 8;  // (16 rows: two waves fetch what the others fetch too)
+#pragma unroll
+  for (int i = 0; i < S::kALoads; ++i) asrc[i] = rows + (size_t)min(r0 + a_first + 8 * i + q8, hi - 1) * K + piece;
+  const bf16_t* wsrc[S::kWLoads];
+#pragma unroll
+  for (int i = 0; i < S::kWLoads; ++i) {
+    const int r = (wave * S::kWLoads + i) * 8 + q8;  // row of the buffer
+    int row;
+    if constexpr (GLU) {
+      const int in = r % S::WN, half = in / (S::WN / 2);
+      row = half * N + min(n0 + (r / S::WN) * (S::WN / 2) + in % (S::WN / 2), N - 1);
+    } else {
+      row = min(n0 + r, N - 1);
+    }
+    wsrc[i] = we + (size_t)row * K + piece;
+  }
+  const uint32_t base = (uint32_t)(uintptr_t)lds_e;
+  const uint32_t a_at = __builtin_amdgcn_readfirstlane(base + a_first * kStepE * 2);
+  const uint32_t w_at = __builtin_amdgcn_readfirstlane(base + (BM + wave * S::kWLoads * 8) * kStepE * 2);
+  auto issue = [&](int step, int buffer) {
+#pragma unroll
+    for (int i = 0; i < S::kALoads; ++i) rows_to_lds(asrc[i] + step * kStepE, a_at + (buffer * S::kStage + i * 8 * kStepE) * 2);
+#pragma unroll
+    for (int i = 0; i < S::kWLoads; ++i) rows_to_lds(wsrc[i] + step * kStepE, w_at + (buffer * S::kStage + i * 8 * kStepE) * 2);
+  };
+
+  float4_e acc[NT][MT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int c = 0; c < MT; ++c) acc[t][c] = float4_e{0.f, 0.f, 0.f, 0.f};
+
+  const int am = (wave % WAVES_M) * S::WM, wn = wave / WAVES_M;
+  const int at[2] = {n16 * kStepE + 8 * (g4 ^ (n16 % 8)), n16 * kStepE + 8 * ((4 + g4) ^ (n16 % 8))};
+  bf16x8_e wop[2][NT], aop[2][MT];
+  auto operands = [&](int buffer, int half) {
+    const bf16_t* as = lds_e + buffer * S::kStage + am * kStepE + at[half];
+    const bf16_t* ws = lds_e + buffer * S::kStage + (BM + wn * S::WN) * kStepE + at[half];
+#pragma unroll
+    for (int c = 0; c < MT; ++c) aop[half][c] = *reinterpret_cast<const bf16x8_e*>(as + c * 16 * kStepE);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) wop[half][t] = *reinterpret_cast<const bf16x8_e*>(ws + t * 16 * kStepE);
+  };
+  auto multiply = [&](int half) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int c = 0; c < MT; ++c) acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wop[half][t], aop[half][c], acc[t][c], 0, 0, 0);
+  };
+
+  // all loads are unconditional (past the end the last step is fetched again and never used), so that a wave's count of
+  // outstanding loads is the same in every trip
+  const int steps = K / kStepE;
+#pragma unroll
+  for (int s = 0; s < kStages - 1; ++s) issue(min(s, steps - 1), s);
+  __builtin_amdgcn_s_waitcnt(S::kWait);
+  __syncthreads();
+  operands(0, 0);
+  int buffer = 0;
+  for (int i = 0; i < steps; ++i) {
+    // (everybody passed the barrier below after reading the last of step i - 1, whose buffer is filled again here)
+    issue(min(i + kStages - 1, steps - 1), buffer == 0 ? kStages - 1 : buffer - 1);
+    operands(buffer, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(0);
+    __builtin_amdgcn_sched_barrier(0);
+    buffer = buffer + 1 == kStages ? 0 : buffer + 1;
+    __builtin_amdgcn_s_waitcnt(S::kWait);  // this wave's loads of step i + 1 have landed; after the barrier everybody's have
+    __syncthreads();
+    operands(buffer, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(1);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // the last, unused fetches must not land after the block has gone
+
+  // acc[t][c][i]: row r0 + am + 16 c + n16, W row 16 t + 4 g4 + i of the wave's
+#pragma unroll
+  for (int c = 0; c < MT; ++c) {
+    const int r = r0 + am + 16 * c + n16;
+    if (r >= hi) continue;
+    if constexpr (GLU) {
+#pragma unroll
+      for (int t = 0; t < NT / 2; ++t) {
+        const int n = n0 + wn * (S::WN / 2) + 16 * t + 4 * g4;
+        if (n >= N) continue;  // (N is a multiple of 4)
+        bf16x4_e out;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float g = acc[t][c][i];
+          out[i] = (__bf16)(g / (1.0f + expf(-g)) * acc[t + NT / 2][c][i]);
+        }
+        *reinterpret_cast<bf16x4_e*>(mid + (size_t)r * N + n) = out;
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const int n = n0 + wn * S::WN + 16 * t + 4 * g4;
+        if (n < N) *reinterpret_cast<float4_e*>(y + (size_t)r * N + n) = acc[t][c];
+      }
+    }
+  }
+}
+
+template <int BM, int BN, int WAVES_M, int kStages, bool GLU>
+int launch_expert_tiles(const void* rows, const void* w, const int32_t* offsets, int n_experts, void* mid, float* y, int K, int N, int pairs,
+                        hipStream_t stream) {
+  using S = ExpertTile<BM, BN, WAVES_M, kStages, GLU>;
+  const auto kernel = expert_tile_kernel<BM, BN, WAVES_M, kStages, GLU>;
+  if (S::kLdsBytes > 48 * 1024) {
+    hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, S::kLdsBytes);
+    if (err != hipSuccess) return tl_fail(TL_ERR_HIP, "expert products: %s", hipGetErrorString(err));
+  }
+  const int n_tiles = (N + S::kColumns - 1) / S::kColumns;
+  const int per_xcd = (n_tiles + kXcds - 1) / kXcds;
+  const int most = (pairs < n_experts ? pairs : n_experts) + pairs / BM;  // row tiles there can be
+  kernel<<<dim3((unsigned)(kXcds * per_xcd) * most), 256, S::kLdsBytes, stream>>>((const bf16_t*)rows, (const bf16_t*)w, offsets, n_experts,
+                                                                               (bf16_t*)mid, y, K, N);
+  return tl_check_launch("expert_tiles");
+}
+
+}  // namespace
+
+// Sizes the kernel takes: K a multiple of a step, columns in fours.
+bool tl_expert_tiles_fit(int K, int N) { return K % kStepE == 0 && N % 4 == 0; }
+
+// mid != null: the gated product (w [E, 2 N, K], gate rows then up rows), otherwise y = the plain one (w [E, N, K]).
+//
+// Which tile: by the rows an expert has on average (`pairs` counts those of outputs that are no experts too).  Measured at
+// 8 experts, gated + plain product in us, widths 4,096 x 3,584 | 2,048 x 2,048, with 16, 32, 64 and 128 rows a tile:
+// 16 pairs 119 120 119 - | 48 48 54 -; 256 pairs (32 rows) 163 137 135 173 | 61 59 55 79; 1,024 pairs (128 rows) - - 227 235
+// | - - 84 87; 2,424 pairs (303 rows) - - 371 364 | - - 127 125; 4,096 pairs - - 592 518 | - - 195 195.  (128 x 256 tiles
+// with one block a CU: 585 at 4,096 pairs.)
+int tl_expert_tiles(const void* rows, const void* w, const int32_t* offsets, int n_experts, void* mid, float* y, int K, int N, int pairs,
+                    hipStream_t stream) {
+  const double mean = (double)pairs / n_experts;
+#define TL_TILES(BM, BN, WM, ST, GLU) return launch_expert_tiles<BM, BN, WM, ST, GLU>(rows, w, offsets, n_experts, mid, y, K, N, pairs, stream)
+  if (mid) {
+    if (mean <= 12) TL_TILES(16, 128, 1, 4, true);
+    if (mean <= 24) TL_TILES(32, 128, 1, 4, true);
+    if (mean <= 256) TL_TILES(64, 128, 1, 3, true);
+    TL_TILES(128, 128, 2, 2, true);
+  }
+  if (mean <= 12) TL_TILES(16, 64, 1, 4, false);
+  if (mean <= 48) TL_TILES(32, 64, 1, 4, false);
+  if (mean <= 128) TL_TILES(64, 128, 1, 3, false);
+  TL_TILES(128, 128, 2, 2, false);
+#undef TL_TILES
+}

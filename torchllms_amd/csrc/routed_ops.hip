@@ -286,7 +286,8 @@ expert_rows_held_kernel(const bf16_t* __restrict__ rows, const bf16_t* __restric
   }
 }
 
-// The same two products on the matrix cores, for experts with many rows: a wave takes 16 outputs of one expert and up
+// The same two products on the matrix cores, for experts with many rows whose widths the tiles of gemm_experts.hip do not
+// take: a wave takes 16 outputs of one expert and up
 // to 32 of its rows at a time, and walks K in steps of 128: a lane asks for four neighbouring 16-byte pieces of its
 // weight row (and of its up row) and of its one or two rows of x, straight from memory (the rows are small and come from
 // the caches; no LDS, no barrier), and every piece is one MFMA 16x16x32 (which k a lane holds does not matter as long as
@@ -761,11 +762,18 @@ static int outputs_per_block(int n_experts, int n_out, int max_rows) {
 }
 
 // rows [pairs, D] in the order of their experts, offsets [n_experts + 1 ..]; mid [pairs, F].
+// (gemm_experts.hip)
+bool tl_expert_tiles_fit(int K, int N);
+int tl_expert_tiles(const void* rows, const void* w, const int32_t* offsets, int n_experts, void* mid, float* y, int K, int N, int pairs,
+                    hipStream_t stream);
+
 TL_EXPORT int tl_expert_glu_rows(const void* rows, const void* w_gu, const int32_t* offsets, int n_experts, void* mid, int D, int F,
                                  int max_rows, int dtype, hipStream_t stream) {
   TL_REQUIRE(n_experts >= 0 && D > 0 && F > 0 && max_rows >= 0, "expert_glu_rows: bad sizes");
   if (n_experts == 0 || max_rows == 0) return TL_OK;
   if (dtype != TL_F32 && dtype != TL_BF16) return tl_fail(TL_ERR_ARG, "expert_glu_rows: unknown dtype %d", dtype);
+  if (dtype == TL_BF16 && tl_expert_tiles_fit(D, F))
+    return tl_expert_tiles(rows, w_gu, offsets, n_experts, mid, nullptr, D, F, max_rows, stream);
   if (dtype == TL_BF16 && D % 8 == 0 && D <= kHeldMaxWidth)
     return launch_rows_held<true>(rows, w_gu, offsets, n_experts, mid, nullptr, D, F, max_rows, stream);
   const int elem = dtype == TL_F32 ? 4 : 2;
@@ -793,6 +801,8 @@ TL_EXPORT int tl_expert_down_rows(const void* mid, const void* w_d, const int32_
   TL_REQUIRE(n_experts >= 0 && D > 0 && F > 0 && max_rows >= 0, "expert_down_rows: bad sizes");
   if (n_experts == 0 || max_rows == 0) return TL_OK;
   if (dtype != TL_F32 && dtype != TL_BF16) return tl_fail(TL_ERR_ARG, "expert_down_rows: unknown dtype %d", dtype);
+  if (dtype == TL_BF16 && tl_expert_tiles_fit(F, D))
+    return tl_expert_tiles(mid, w_d, offsets, n_experts, nullptr, y, F, D, max_rows, stream);
   if (dtype == TL_BF16 && F % 8 == 0 && F <= kHeldMaxWidth)
     return launch_rows_held<false>(mid, w_d, offsets, n_experts, nullptr, y, F, D, max_rows, stream);
   const int elem = dtype == TL_F32 ? 4 : 2;

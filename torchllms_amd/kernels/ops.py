@@ -133,6 +133,7 @@ from .routed_ops import (  # noqa: F401
     expert_gather,
     expert_glu_rows,
     expert_pair_products,
+    expert_tiles_fit,
     PAIR_PRODUCTS_MOST,
     pair_norm_add_norm,
     post_norm_add_norm,

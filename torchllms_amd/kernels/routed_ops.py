@@ -66,10 +66,15 @@ def _expert_rows(rows, weights, offsets, what):
         raise KernelError(f"{what}: offsets must be contiguous int32 with an entry per expert and one more")
 
 
+def expert_tiles_fit(width: int, expert_size: int) -> bool:
+    """Do tiles on the matrix cores serve both products of experts of these sizes in bfloat16, however many rows there are?"""
+    return width % 64 == 0 and expert_size % 64 == 0
+
+
 def expert_glu_rows(rows: torch.Tensor, w_gate_up: torch.Tensor, offsets: torch.Tensor) -> torch.Tensor:
     """``mid[r] = silu(Wg[e] rows[r]) * (Wu[e] rows[r])`` for the rows ``offsets[e] .. offsets[e + 1]`` of every expert
     ``e`` of ``w_gate_up`` [E, 2F, D] (gate rows, then up rows); ``rows`` [pairs, D] as ``expert_gather`` leaves them.
-    An expert's weights are read once for up to eight of its rows.  Returns [pairs, F]; rows behind ``offsets[E]`` (pairs of
+    An expert's weights are read once for a tile of its rows.  Returns [pairs, F]; rows behind ``offsets[E]`` (pairs of
     outputs that are no experts) are left unwritten."""
     _gpu(rows, w_gate_up, offsets)
     _expert_rows(rows, w_gate_up, offsets, "expert_glu_rows")

@@ -116,16 +116,17 @@ class RoutedExperts(FeedForward):
     works on instead of what comes out.
 
     A token's result depends on nothing but the token.  The (token, choice) pairs of a step are put in the order of
-    their experts on the device, and a kernel walks every expert's rows with the expert's weights read once for eight
+    their experts on the device, and a kernel walks every expert's rows with the expert's weights read once for a tile
     of them; each row's sums have an order of their own, so in 32-bit a token's result has the same bits in every
-    step, and the launches are fixed by the step's shape (decode steps are replayed from graphs).  A bfloat16 step
-    that brings prompts and has ``GROUPED_FROM`` pairs or more runs one matrix product per expert over its rows
-    instead; for that the host reads how many rows each expert got, once a layer.  A bfloat16 step of at most
+    step, and the launches are fixed by the step's shape (decode steps are replayed from graphs).  Widths that the
+    tiles do not take (``ops.expert_tiles_fit``): a bfloat16 step that brings prompts and has ``GROUPED_FROM`` pairs or
+    more runs one library product per expert over its rows; for that the host reads how many rows each expert got, once
+    a layer.  A bfloat16 step of at most
     ``ops.PAIR_PRODUCTS_MOST`` pairs (one or two requests decoding) gathers nothing: every pair runs through the dense
     layers' weight-streaming products, which read on the device which expert's matrix is meant."""
 
     graph_safe = True
-    #: (token, choice) pairs of a bfloat16 step with prompts from which on the experts run as matrix products
+    #: (token, choice) pairs of a bfloat16 step with prompts from which on experts of other widths run as library products
     GROUPED_FROM = 512
 
     def __init__(self, hidden_size: int, expert_size: int, num_experts: int, top: int, num_identity: int = 0, shared_size: int = 0,
@@ -222,7 +223,8 @@ class RoutedExperts(FeedForward):
             y = ops.expert_pair_products(x, self.w_gu, self.w_down, ids, input_weights=inputs)
             return ops.expert_combine(y, self._own_rows(x.shape[0], x.device), ids, weights, self.E, x, shared, gate)
         rows, pos, offsets = ops.expert_gather(x, ids, n_out, input_weights=inputs)
-        if x.dtype == torch.float32 or ctx.host.max_q_len <= 1 or x.shape[0] * self.top < self.GROUPED_FROM:
+        if (x.dtype == torch.float32 or ops.expert_tiles_fit(self.hidden_size, self.F) or ctx.host.max_q_len <= 1
+                or x.shape[0] * self.top < self.GROUPED_FROM):
             y = ops.expert_down_rows(ops.expert_glu_rows(rows, self.w_gu, offsets), self.w_down, offsets)
             return ops.expert_combine(y, pos, ids, weights, self.E, x, shared, gate)
         bounds = offsets.tolist()  # (the one place a step with prompts waits for the GPU)
