@@ -355,6 +355,36 @@ def test_gemm_f32_tiles_give_the_bits_of_the_kernel_for_few_rows(m, n, k, aligne
         assert torch.equal(_ops().gemm_f32(x[first : first + 9], w), got[first : first + 9])
 
 
+# ----------------------------------------------------------------------------- layer norm
+@pytest.mark.parametrize("hidden", [4, 5, 1020, 1024, 1028, 2052, 4096, 8192, 8196])
+@pytest.mark.parametrize("stream, out", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16), (torch.bfloat16, torch.bfloat16)])
+def test_layernorm_of_every_width(hidden, stream, out):
+    """Rows held in registers (multiples of 4 up to 8,192, whole and partly filled) and rows through LDS; no, one and two
+    terms added, the sum returned in place, rows gathered; a row's bits do not depend on the rows beside it."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(hidden)
+    x = (torch.randn(5, hidden, generator=g) * 3 + 1).to(stream)
+    terms = [torch.randn(5, hidden, generator=g).to(out) for _ in range(2)]
+    w, b = torch.randn(hidden, generator=g), torch.randn(hidden, generator=g)
+    rows = torch.tensor([3, 0], dtype=torch.int32)
+    for count in (0, 1, 2):
+        delta = ops.ScaledSum([t.to(DEV) for t in terms[:count]], 0.5) if count else None
+        h = x.double() + (0.5 * sum(t.double() for t in terms[:count]) if count else 0.0)
+        if stream == torch.bfloat16 and count:
+            h = (x.float() + 0.5 * sum(t.float() for t in terms[:count])).bfloat16().double()
+        c = h - h.mean(-1, keepdim=True)
+        want = c / torch.sqrt((c * c).mean(-1, keepdim=True) + 1e-5) * w.double() + b.double()
+        y = ops.layernorm(x.to(DEV), w.to(DEV), b.to(DEV), 1e-5, out, delta=delta)
+        # the row's sum and squares: hidden roundings at most, seen through a factor of about one; one rounding of the result
+        tol = (2.0 ** -8 if out == torch.bfloat16 else 0.0) + 2.0 ** -20
+        assert bool(((y.cpu().double() - want).abs() <= tol * (want.abs() + 4.0)).all())
+        alone = ops.layernorm(x.to(DEV), w.to(DEV), b.to(DEV), 1e-5, out, delta=delta, rows=rows.to(DEV))
+        assert torch.equal(alone, y[rows.long().to(DEV)])
+        if count:
+            s, z = ops.layernorm(x.to(DEV), w.to(DEV), b.to(DEV), 1e-5, out, delta=delta, return_sum=True)
+            assert torch.equal(z, y) and bool(((s.cpu().double() - h).abs() <= 2.0 ** -22 * (h.abs() + 1)).all())
+
+
 # ----------------------------------------------------------------------------- routed experts' products by tiles
 @pytest.mark.parametrize("counts, D, F", [
     ([1], 64, 64), ([0, 3, 0, 17, 1, 0], 128, 192), ([15, 16, 17, 33], 64, 320), ([31, 0, 32, 65], 192, 64), ([64, 63, 129, 0, 65], 128, 448),
