@@ -111,7 +111,7 @@ layernorm_kernel(const HT* x, const T* __restrict__ d0, const T* __restrict__ d1
 // The same for rows of a multiple of 4 elements, up to 8,192: a thread holds its part of the row in registers, four
 // elements a load, and asks for all of it (and for its part of w and b) before it looks at any.  (In the kernel above the
 // rows may be written where they are read, so every trip of the loop waits for its loads: one row of 4,096 took 19 us of
-// a decode step, 4.5 here; 2,048 rows 29, 22 here = 4.9 TB/s.)  The order of the sums depends on the width alone.
+// a decode step, 5.6 here; 2,048 rows 29, 25 here = 4.4 TB/s.)  The order of the sums depends on the width alone.
 template <typename HT, typename T, int CH>
 __global__ void __launch_bounds__(kNormThreads)
 layernorm_held_kernel(const HT* x, const T* __restrict__ d0, const T* __restrict__ d1, float mult,
@@ -1315,11 +1315,23 @@ TL_EXPORT int tl_selective_scan(const void* x, const void* dt_pre, int dt_dtype,
 // gate (proj itself, or a tensor of its own); gate_sigmoid: the gate's activation is the logistic function, not silu.
 // a_ch (or null): 32-bit pre-activations of a decay per key channel, [n_tokens, a_stride] with H * dk columns; then
 // dt_bias has H * dk entries.
+// (delta_chunks.hip) Returns 1, with nothing launched, for sizes and alignments that the chunks do not take.
+int tl_delta_chunks(const void* qkv, int stride, const void* proj, int proj_stride, int b_off, int a_off, const float* A_log, const float* dt_bias,
+                    float* state, long long state_stride, const int32_t* qo_indptr, const int32_t* slot_ids, float* o_raw, int t_first, int t_last,
+                    int rows, int H, int G, int dk, int dv, const float* a_ch, int a_stride, float plain_rate, float* ws, long long floats,
+                    hipStream_t stream);
+int tl_memory_chunks(const void* proj, int stride, int q_off, int k_off, int v_off, int i_off, int f_off, const float* i_bias, const float* f_bias,
+                     float cap, float* state, long long state_stride, const int32_t* qo_indptr, const int32_t* slot_ids, float* o_raw, float* den,
+                     int t_first, int t_last, int rows, int H, int dk, int dv, float* ws, long long floats, hipStream_t stream);
+
+// ws (ws_floats of tl_chunk_floats): a bfloat16 step's first single_rows rows, one token each, take the kernel for such
+// rows, the others go by chunks of tokens on the matrix cores, if sizes and alignments allow it.
 TL_EXPORT int tl_gated_delta(const void* qkv, int qkv_stride, const void* proj, int proj_stride, int gate_off, int b_off,
                              int a_off, const float* A_log, const float* dt_bias, const float* norm_w, float eps, float* state,
                              long long state_stride, const int32_t* qo_indptr, const int32_t* slot_ids, void* out, int n_tokens,
                              int n_seqs, int H, int G, int dk, int dv, float* o_raw, int dtype, const void* gate, int gate_stride,
-                             int gate_sigmoid, const float* a_ch, int a_stride, float plain_rate, hipStream_t stream) {
+                             int gate_sigmoid, const float* a_ch, int a_stride, float plain_rate, float* ws, long long ws_floats,
+                             int single_rows, hipStream_t stream) {
   TL_REQUIRE(n_seqs >= 0 && n_tokens >= 0 && H > 0 && G > 0 && dk > 0 && dv > 0, "gated_delta: bad sizes");
   TL_REQUIRE(H % G == 0, "gated_delta: %d heads are not a multiple of %d key heads", H, G);
   if (dk > 256) return tl_fail(TL_ERR_UNSUPPORTED, "gated_delta: keys of %d channels, at most 256", dk);
@@ -1332,17 +1344,27 @@ TL_EXPORT int tl_gated_delta(const void* qkv, int qkv_stride, const void* proj, 
   int lpc = 1;
   while (rows * lpc < dk) lpc *= 2;  // at most 16: a column's lanes lie in one row of 16 lanes
   // columns a block: 16 while that leaves fewer than two blocks a CU, else 32 (a step of single tokens: always 32)
-  const bool single = n_tokens == n_seqs;
   const bool ch = a_ch != nullptr;
   const bool plain = plain_rate > 0.f;
   TL_REQUIRE(!plain || ch, "gated_delta: the plain rule has a decay per key channel");
   TL_REQUIRE(plain || (A_log != nullptr && proj != nullptr), "gated_delta: no A_log or no projections");
+  TL_REQUIRE(single_rows >= 0 && single_rows <= n_seqs, "gated_delta: %d rows of one token among %d", single_rows, n_seqs);
+  bool chunked = false;
+  if (ws != nullptr && dtype == TL_BF16 && n_tokens > n_seqs) {
+    const int rc = tl_delta_chunks(qkv, qkv_stride, proj, proj_stride, b_off, a_off, A_log, dt_bias, state, state_stride, qo_indptr + single_rows,
+                                   slot_ids + single_rows, o_raw, single_rows, n_tokens, n_seqs - single_rows, H, G, dk, dv, a_ch, a_stride,
+                                   plain_rate, ws, ws_floats, stream);
+    if (rc != 1 && rc != TL_OK) return rc;
+    chunked = rc == TL_OK;
+  }
+  const int walked = chunked ? single_rows : n_seqs;  // rows that are walked token by token
+  const bool single = chunked || n_tokens == n_seqs;
   const int cols = !single && (long long)n_seqs * H * ((dv + 15) / 16) < 2LL * tl_device_facts().compute_units ? 16 : 32;
   const int threads = (cols * lpc + kWave - 1) / kWave * kWave;
   const int col_groups = (dv + cols - 1) / cols;
   const int dkp = dk + dk / 16 * 4;
   const size_t lds = ((size_t)kDeltaTile * (2 * dkp + 2 * cols + 6 + (ch ? dkp : 0))) * sizeof(float);
-  const dim3 grid(H * col_groups, n_seqs);
+  const dim3 grid(H * col_groups, walked);
 #define TL_DELTA_R(T, VEC, R, C, CH)                                                                                   \
   gated_delta_kernel<T, VEC, R, C, CH><<<grid, threads, lds, stream>>>(                                                \
       (const T*)qkv, qkv_stride, (const T*)proj, proj_stride, b_off, a_off, A_log, dt_bias, state, state_stride,       \
@@ -1382,8 +1404,10 @@ TL_EXPORT int tl_gated_delta(const void* qkv, int qkv_stride, const void* proj, 
     else if (ch) TL_DELTA_ANY(T, false, 1);      \
     else TL_DELTA_ANY(T, false, 0);              \
   } while (0)
-  if (dtype == TL_F32) TL_DELTA_T(float);
-  else TL_DELTA_T(bf16_t);
+  if (walked > 0) {
+    if (dtype == TL_F32) TL_DELTA_T(float);
+    else TL_DELTA_T(bf16_t);
+  }
 #undef TL_DELTA_T
 #undef TL_DELTA_ANY
 #undef TL_DELTA_STEP
@@ -1696,7 +1720,8 @@ TL_EXPORT int tl_matrix_memory(const void* proj, int stride, int q_off, int k_of
                                const float* i_bias, const float* f_bias, float cap, const void* gate, int gate_stride,
                                int gate_off, const float* norm_w, float eps, float* state, long long state_stride,
                                const int32_t* qo_indptr, const int32_t* slot_ids, void* out, int n_tokens, int n_seqs, int H,
-                               int dk, int dv, float* o_raw, float* den, int dtype, hipStream_t stream) {
+                               int dk, int dv, float* o_raw, float* den, int dtype, float* ws, long long ws_floats, int single_rows,
+                               hipStream_t stream) {
   TL_REQUIRE(n_seqs >= 0 && n_tokens >= 0 && H > 0 && dk > 0 && dv > 0 && cap > 0.f, "matrix_memory: bad sizes");
   if (dk > 256) return tl_fail(TL_ERR_UNSUPPORTED, "matrix_memory: keys of %d channels, at most 256", dk);
   TL_REQUIRE(n_seqs <= 65535 && n_tokens <= 0x7fffffff / 4, "matrix_memory: too many requests or tokens a step");
@@ -1710,9 +1735,19 @@ TL_EXPORT int tl_matrix_memory(const void* proj, int stride, int q_off, int k_of
   const int col_groups = (dv + 1 + kMemCols - 1) / kMemCols;
   const int dkp = dk + dk / 16 * 4;
   const size_t lds = ((size_t)kDeltaTile * (2 * dkp + 2 * kMemCols + 4) + 4) * sizeof(float);
-  const dim3 grid(H * col_groups, n_seqs);
+  TL_REQUIRE(single_rows >= 0 && single_rows <= n_seqs, "matrix_memory: %d rows of one token among %d", single_rows, n_seqs);
+  bool chunked = false;  // (see tl_gated_delta)
+  if (ws != nullptr && dtype == TL_BF16 && n_tokens > n_seqs) {
+    const int rc = tl_memory_chunks(proj, stride, q_off, k_off, v_off, i_off, f_off, i_bias, f_bias, cap, state, state_stride,
+                                    qo_indptr + single_rows, slot_ids + single_rows, o_raw, den, single_rows, n_tokens, n_seqs - single_rows, H,
+                                    dk, dv, ws, ws_floats, stream);
+    if (rc != 1 && rc != TL_OK) return rc;
+    chunked = rc == TL_OK;
+  }
+  const int walked = chunked ? single_rows : n_seqs;
+  const dim3 grid(H * col_groups, walked);
   const bool vec = dk % 4 == 0 && ((uintptr_t)state % 16) == 0 && state_stride % 4 == 0;
-  const bool single = n_tokens == n_seqs;
+  const bool single = chunked || n_tokens == n_seqs;
   const size_t step_lds = 2 * (size_t)dkp * sizeof(float);
 #define TL_MEM(T, VEC, R)                                                                                               \
   do {                                                                                                                  \
@@ -1732,8 +1767,10 @@ TL_EXPORT int tl_matrix_memory(const void* proj, int stride, int q_off, int k_of
     else if (rows == 8) TL_MEM(T, false, 8);         \
     else TL_MEM(T, false, 16);                       \
   } while (0)
-  if (dtype == TL_F32) TL_MEM_T(float);
-  else TL_MEM_T(bf16_t);
+  if (walked > 0) {
+    if (dtype == TL_F32) TL_MEM_T(float);
+    else TL_MEM_T(bf16_t);
+  }
 #undef TL_MEM_T
 #undef TL_MEM
   int rc = tl_check_launch("matrix_memory");

@@ -30,6 +30,7 @@ CORE_NAME = "torchllms_amd_core"
 CORE_SOURCES = [
     "elementwise.hip",
     "attention_generic.hip",
+    "delta_chunks.hip",
     "gemm_experts.hip",
     "gemm_f32.hip",
     "gemm_stream.hip",

@@ -7,7 +7,7 @@ an exception is raised.
 from __future__ import annotations
 
 import ctypes
-from ctypes import c_char_p, c_float, c_int, c_int64, c_uint64, c_void_p
+from ctypes import c_char_p, c_float, c_int, c_int64, c_longlong, c_uint64, c_void_p
 from typing import Dict, Optional
 
 from . import build as _build
@@ -40,8 +40,8 @@ _CORE_SIGNATURES = {
     "tl_rope_norm_kv_write": [_P, _I, _I, _I, _I, _I, _P, _I, _I, _F, _P, _P, _P, _I, _I, _P],
     "tl_causal_conv": [_P, _I, _P, _P, _P, _I64, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
     "tl_selective_scan": [_P, _P, _I, _P, _I, _I, _I, _P, _I, _P, _P, _P, _P, _I64, _P, _P, _P, _I, _I, _I, _I, _P, _P, _I, _P, _P, _P],
-    "tl_gated_delta": [_P, _I, _P, _I, _I, _I, _I, _P, _P, _P, _F, _P, _I64, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _P, _I, _I, _P, _I, _F, _P],
-    "tl_matrix_memory": [_P, _I, _I, _I, _I, _I, _I, _P, _P, _F, _P, _I, _I, _P, _F, _P, _I64, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _I, _P],
+    "tl_gated_delta": [_P, _I, _P, _I, _I, _I, _I, _P, _P, _P, _F, _P, _I64, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _P, _I, _I, _P, _I, _F, _P, _I64, _I, _P],
+    "tl_matrix_memory": [_P, _I, _I, _I, _I, _I, _I, _P, _P, _F, _P, _I, _I, _P, _F, _P, _I64, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _I, _P, _I64, _I, _P],
     "tl_router_topk": [_P, _I, _P, _I, _I, _I, _P, _P, _I, _I, _I, _F, _P, _I, _P],
     "tl_streams_update": [_P, _I, _I64, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P],
     "tl_streams_open": [_P, _P, _I, _I64, _P],
@@ -110,6 +110,8 @@ def core() -> ctypes.CDLL:
     if _core is None:
         path = _build.build_core()
         lib = ctypes.CDLL(str(path))
+        lib.tl_chunk_floats.restype = c_longlong  # (a count, not a status)
+        lib.tl_chunk_floats.argtypes = [c_int] * 5
         lib.tl_last_error.restype = c_char_p
         lib.tl_last_error.argtypes = []
         _declare(lib, _CORE_SIGNATURES)

@@ -310,6 +310,23 @@ def selective_scan(
     return out
 
 
+#: the longest row of a step from which on prompts' rows of a bfloat16 step go by chunks of 16 tokens, and the most 32-bit
+#: numbers a step takes for that (a gigabyte: a step of so many rows is walked)
+CHUNKS_FROM, CHUNK_FLOATS_MOST = 16, 1 << 28
+
+
+def _chunk_workspace(dtype: torch.dtype, longest: int, single_rows: int, n: int, n_seqs: int, n_heads: int, head_dim: int, device, memory: bool = False):
+    """``(workspace or None, its size)`` of a step whose longest row brings ``longest`` tokens."""
+    if not 0 <= single_rows <= n_seqs:
+        raise KernelError(f"{single_rows} rows of one token among {n_seqs} rows")
+    if dtype != torch.bfloat16 or longest < CHUNKS_FROM or n <= n_seqs:
+        return None, 0
+    floats = core().tl_chunk_floats(n - single_rows, n_seqs - single_rows, n_heads, head_dim, 1 if memory else 0)
+    if not 0 < floats <= CHUNK_FLOATS_MOST:
+        return None, 0
+    return torch.empty(floats, dtype=torch.float32, device=device), floats
+
+
 def gated_delta(
     qkv: torch.Tensor,
     proj: torch.Tensor,
@@ -331,6 +348,8 @@ def gated_delta(
     gate: Optional[torch.Tensor] = None,
     gate_act: str = "silu",
     channel_decay: Optional[torch.Tensor] = None,
+    longest: int = 0,
+    single_rows: int = 0,
 ) -> torch.Tensor:
     """The gated delta rule over each request's tokens, in 32-bit.  ``qkv`` [n, 2 G dk + H dv]: query
     heads | key heads | value heads, already convolved and activated.  Of ``proj`` [n, ..] the output
@@ -344,7 +363,11 @@ def gated_delta(
     ``gate_act`` "sigmoid": the gate is the logistic function of them, not silu.  ``channel_decay`` float32
     [n, H * dk]: every key channel of a head (row of S) has a decay of its own,
     ``exp(-exp(A_log[h]) softplus(channel_decay[t, h, i] + dt_bias[h, i]))`` with ``dt_bias`` of H * dk entries;
-    the column ``a_offset`` of ``proj`` is then not read."""
+    the column ``a_offset`` of ``proj`` is then not read.
+
+    ``longest``: the tokens of the step's longest row.  From ``CHUNKS_FROM`` on, in bfloat16 and for keys of 64 or 128
+    channels, the rows behind the first ``single_rows`` (which bring one token each) go by chunks of 16 tokens on the
+    32-bit matrix cores, with sums in another order than the walk's."""
     _gpu(qkv, proj, A_log, dt_bias, norm_weight, gate, channel_decay)
     H, G, dk, dv = n_heads, n_key_heads, head_dim, v_head_dim
     n = qkv.shape[0]
@@ -367,6 +390,7 @@ def gated_delta(
             raise KernelError(f"gated_delta: a float32 vector of {size} entries expected, got {tuple(v.shape)} {v.dtype}")
     n_seqs = _step_rows(None, qo_indptr, slot_ids, n, state)
     region, stride = state_region(state, state_offset, H * dv * dk)
+    ws, floats = _chunk_workspace(qkv.dtype, longest, single_rows, n, n_seqs, H, dk, qkv.device)
     out = torch.empty((n, H * dv), dtype=qkv.dtype, device=qkv.device)
     o_raw = torch.empty((n, H * dv), dtype=torch.float32, device=qkv.device)
     check(
@@ -375,7 +399,7 @@ def gated_delta(
             dt_bias.data_ptr(), norm_weight.data_ptr(), float(eps), region, stride, qo_indptr.data_ptr(), slot_ids.data_ptr(),
             out.data_ptr(), n, n_seqs, H, G, dk, dv, o_raw.data_ptr(), dtype_code(qkv.dtype), gate_src.data_ptr(), gate_src.stride(0),
             1 if gate_act == "sigmoid" else 0, _ptr(channel_decay), channel_decay.stride(0) if channel_decay is not None else 0,
-            0.0, _stream(),
+            0.0, _ptr(ws), floats, single_rows, _stream(),
         )
     )
     return out
@@ -397,13 +421,16 @@ def gated_linear(
     n_heads: int,
     head_dim: int,
     v_head_dim: int,
+    longest: int = 0,
+    single_rows: int = 0,
 ) -> torch.Tensor:
     """Gated linear attention over each request's tokens, in 32-bit.  ``qkv`` [n, 2 H dk + H dv]: query heads | key
     heads | value heads as projected.  Per head, with q times dk^-1/2 and a decay for every key channel
     ``alpha = sigmoid(decay_pre[t, h, i] + decay_bias[h, i]) ** decay_power`` (``decay_pre`` float32 [n, H * dk]):
     ``S <- diag(alpha) S + k v^T; o = S^T q``; then o over its root mean square, times ``norm_weight`` [dv], times
     silu of the gate (H dv columns of ``gate`` from ``gate_offset``).  ``S`` lives at ``state_offset`` of the request's
-    state row, H * dv * dk floats.  Returns [n, H * dv].  The recurrence is the delta rule's kernel with its plain rule."""
+    state row, H * dv * dk floats.  Returns [n, H * dv].  The recurrence is the delta rule's kernel with its plain rule.
+    ``longest``, ``single_rows``: as ``gated_delta``'s."""
     _gpu(qkv, decay_pre, decay_bias, gate, norm_weight)
     H, dk, dv = n_heads, head_dim, v_head_dim
     n = qkv.shape[0]
@@ -420,6 +447,7 @@ def gated_linear(
         raise KernelError("gated_linear: the decay's power must be positive")
     n_seqs = _step_rows(None, qo_indptr, slot_ids, n, state)
     region, stride = state_region(state, state_offset, H * dv * dk)
+    ws, floats = _chunk_workspace(qkv.dtype, longest, single_rows, n, n_seqs, H, dk, qkv.device)
     out = torch.empty((n, H * dv), dtype=qkv.dtype, device=qkv.device)
     o_raw = torch.empty((n, H * dv), dtype=torch.float32, device=qkv.device)
     check(
@@ -427,7 +455,7 @@ def gated_linear(
             qkv.data_ptr(), qkv.stride(0), None, 0, gate_offset, 0, 0, None, decay_bias.data_ptr(), norm_weight.data_ptr(), float(eps),
             region, stride, qo_indptr.data_ptr(), slot_ids.data_ptr(), out.data_ptr(), n, n_seqs, H, H, dk, dv, o_raw.data_ptr(),
             dtype_code(qkv.dtype), gate.data_ptr(), gate.stride(0), 0, decay_pre.data_ptr(), decay_pre.stride(0), float(decay_power),
-            _stream(),
+            _ptr(ws), floats, single_rows, _stream(),
         )
     )
     return out
@@ -459,6 +487,8 @@ def matrix_memory(
     n_heads: int,
     head_dim: int,
     v_head_dim: int,
+    longest: int = 0,
+    single_rows: int = 0,
 ) -> torch.Tensor:
     """The matrix memory of an mLSTM layer over each request's tokens, in 32-bit.  Of ``proj`` [n, ..] the columns of
     q and k (H heads of dk each), v and the output gate (H heads of dv) and the pre-activations of the input and the
@@ -467,7 +497,7 @@ def matrix_memory(
     ``m' = max(f + m, i); C <- exp(f + m - m') C + exp(i - m') k v^T``, n likewise with k alone,
     ``o = C^T q dk^-1/2 / (max(|n . q dk^-1/2|, exp(-m')) + 1e-6)``; then o over its root mean square, times
     ``norm_weight`` [H * dv], times sigmoid(gate).  C, n and m live at ``state_offset`` of the request's state row
-    (``matrix_memory_state_size`` floats).  Returns [n, H * dv]."""
+    (``matrix_memory_state_size`` floats).  Returns [n, H * dv].  ``longest``, ``single_rows``: as ``gated_delta``'s."""
     _gpu(proj, i_bias, f_bias, norm_weight)
     H, dk, dv = n_heads, head_dim, v_head_dim
     n = proj.shape[0]
@@ -485,6 +515,7 @@ def matrix_memory(
         raise KernelError("matrix_memory: the gates' cap must be positive")
     n_seqs = _step_rows(None, qo_indptr, slot_ids, n, state)
     region, stride = state_region(state, state_offset, matrix_memory_state_size(H, dk, dv))
+    ws, floats = _chunk_workspace(proj.dtype, longest, single_rows, n, n_seqs, H, dk, proj.device, memory=True)
     out = torch.empty((n, H * dv), dtype=proj.dtype, device=proj.device)
     o_raw = torch.empty((n, H * dv), dtype=torch.float32, device=proj.device)
     den = torch.empty((n, H), dtype=torch.float32, device=proj.device)
@@ -493,7 +524,7 @@ def matrix_memory(
             proj.data_ptr(), proj.stride(0), q_offset, k_offset, v_offset, i_offset, f_offset, i_bias.data_ptr(), f_bias.data_ptr(),
             float(gate_cap), proj.data_ptr(), proj.stride(0), gate_offset, norm_weight.data_ptr(), float(eps), region, stride,
             qo_indptr.data_ptr(), slot_ids.data_ptr(), out.data_ptr(), n, n_seqs, H, dk, dv, o_raw.data_ptr(), den.data_ptr(),
-            dtype_code(proj.dtype), _stream(),
+            dtype_code(proj.dtype), _ptr(ws), floats, single_rows, _stream(),
         )
     )
     return out

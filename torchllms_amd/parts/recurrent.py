@@ -199,7 +199,8 @@ class GatedDelta(Mixer):
             channel = ops.linear(proj[:, a_at : a_at + self.decay_rank], self.w_a2, out_dtype=torch.float32)
         y = ops.gated_delta(qkv, proj, gate_at, b_at, a_at, self.A_log, self.dt_bias, self.norm_w, self.norm_eps, state,
                             (self.taps - 1) * c, ctx.qo_indptr, ctx.slot_ids, self.H, self.G, self.dk, self.dv,
-                            gate=gate, gate_act=self.gate_act, channel_decay=channel)
+                            gate=gate, gate_act=self.gate_act, channel_decay=channel, longest=ctx.host.max_q_len,
+                            single_rows=ctx.host.n_decode)
         return ops.linear_to_sum(y, self.w_o)
 
 
@@ -258,7 +259,7 @@ class MatrixMemory(Mixer):
         proj = ops.linear(ops.resolved(x), self.w_all)
         y = ops.matrix_memory(proj, 0, qk, 2 * qk, 2 * qk + 2 * v, 2 * qk + 2 * v + self.H, 2 * qk + v, self.i_b, self.f_b,
                               self.gate_cap, self.norm_w, self.norm_eps, cache.tensor, 0, ctx.qo_indptr, ctx.slot_ids,
-                              self.H, self.dk, self.dv)
+                              self.H, self.dk, self.dv, longest=ctx.host.max_q_len, single_rows=ctx.host.n_decode)
         return ops.linear_to_sum(y, self.w_o)
 
 
@@ -316,7 +317,8 @@ class GatedLinearAttention(Mixer):
         proj = ops.linear(ops.resolved(x), self.w_all)
         pre = ops.linear(proj[:, c + v : c + v + self.rank], self.w_a2, out_dtype=torch.float32)
         y = ops.gated_linear(proj[:, :c], pre, self.a_bias, 1.0 / self.tau, proj, c, self.norm_w, self.norm_eps, cache.tensor, 0,
-                             ctx.qo_indptr, ctx.slot_ids, self.H, self.dk, self.dv)
+                             ctx.qo_indptr, ctx.slot_ids, self.H, self.dk, self.dv, longest=ctx.host.max_q_len,
+                             single_rows=ctx.host.n_decode)
         return ops.linear_to_sum(y, self.w_o)
 
 
