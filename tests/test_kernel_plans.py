@@ -33,6 +33,13 @@ def test_decode_splits_cover_the_range_and_stay_under_a_cu_s_share_of_blocks():
     assert ops.plan_decode_splits(8, 4, 8192, 256) == (1024, 8)
 
 
+def test_short_uneven_requests_in_numbers_are_left_whole():
+    assert ops.decode_splits(64, 8, 1024, 128, uneven=True) == (1024, 1) and ops.decode_splits(64, 8, 768, 64, uneven=True) == (768, 1)
+    for args in ((64, 8, 1025, 128), (63, 8, 1024, 128), (64, 4, 1000, 64), (8, 8, 300, 128)):  # longer, or fewer pairs: as planned
+        assert ops.decode_splits(*args, uneven=True) == ops.plan_decode_splits(*args, uneven=True)
+        assert ops.decode_splits(*args) == ops.plan_decode_splits(*args)
+
+
 def test_a_sampled_row_is_cut_only_when_rows_are_few_and_long():
     assert ops.sample_chunks(1, 128256) == 15 and ops.sample_chunks(8, 128256) == 15
     assert ops.sample_chunks(64, 128256) == 4 and ops.sample_chunks(256, 128256) == 1

@@ -90,6 +90,7 @@ from .attention_ops import (  # noqa: F401
     attention_generic_split,
     attention_prefill,
     decode_attention_supported,
+    decode_splits,
     plan_decode_splits,
     prefill_attention_supported,
     prefill_key_groups,
