@@ -608,6 +608,41 @@ def test_attention_window_edge(dtype, window):
     assert (got[-1].view(hq, dh) - v[inside, 0]).abs().max() < (1e-3 if dtype == torch.float32 else 3e-2)
 
 
+@pytest.mark.parametrize("odd_value", [False, True])
+@pytest.mark.parametrize(
+    "hq, hkv, dh, page, sizes, kw",
+    [(8, 2, 64, 16, [(200, 130), (70, 70), (300, 5), (65, 2)], {}), (4, 4, 128, 5, [(150, 33)], dict(window=40)),
+     (16, 2, 32, 8, [(64, 64), (129, 65)], dict(chunk=48, softcap=3.0)), (6, 3, 16, 3, [(100, 37), (20, 20)], dict(slopes=True)),
+     (3, 1, 128, 16, [(90, 41)], dict(window=64, sinks=True)), (4, 1, 64, 16, [(140, 63)], dict(distances=True))],
+)
+def test_attention_generic_on_the_matrix_cores_gives_the_same_bits(hq, hkv, dh, page, sizes, kw, odd_value):
+    """Prompts of 32-bit models (on_end) take blocks of 64 keys through matrix instructions, in the order of the sums of the
+    kernels that multiply one by one: every form that is accepted, groups of 1, 2, 3, 4 and 8 query heads, tokens that fill no
+    block, several requests in one.  A value that is not a number reaches the queries that see its key and no others."""
+    torch.manual_seed(dh + page)
+    kw = dict(kw)
+    window = kw.pop("window", 0)
+    for name, shape in (("slopes", (hq,)), ("sinks", (hq,)), ("distances", (hq, 50))):
+        if kw.pop(name, False):
+            kw[name] = torch.rand(shape, device=DEV)
+    width = max(-(-S // page) for S, _ in sizes)
+    tables = torch.randperm(width * len(sizes)).view(len(sizes), width)
+    k_pages, v_pages = (torch.randn(width * len(sizes), hkv, page, dh, device=DEV) for _ in range(2))
+    if odd_value:
+        S, sq = sizes[0]
+        at = S - sq // 2
+        v_pages[int(tables[0, at // page]), 0, at % page, 3] = float("nan")
+        v_pages[int(tables[0, (at + 3) // page]), 0, (at + 3) % page, 5] = float("inf")
+    seqs = [r for r, (S, sq) in enumerate(sizes) for _ in range(sq)]
+    poss = [p for S, sq in sizes for p in range(S - sq, S)]
+    q = torch.randn(len(seqs), hq * dh + 12, device=DEV)
+    args = (q, hq, hkv, dh, k_pages, v_pages, _i32(seqs), _i32(poss), _i32(tables.tolist()), window, dh ** -0.5)
+    want, got = (_ops().attention_generic(*args, on_end=on_end, **kw) for on_end in (False, True))
+    assert torch.equal(torch.isnan(want), torch.isnan(got))
+    assert bool(torch.isnan(want).any()) == odd_value
+    assert torch.equal(want.nan_to_num(7.0), got.nan_to_num(7.0))
+
+
 def test_attention_window_never_reads_released_pages():
     """Blocks wholly before the window are -1 in the block table; the kernel must not touch them."""
     torch.manual_seed(0)

@@ -15,6 +15,7 @@
 #include <limits.h>
 
 #include "common.h"
+#include "recurrence.h"  // mfma_f32
 
 namespace {
 
@@ -448,6 +449,246 @@ attention_tile_kernel(const T* __restrict__ q, int q_stride, T* __restrict__ out
   }
 }
 
+// The same result again for the prompts of 32-bit models, on the matrix cores: v_mfma_f32_16x16x4_f32 is a chain of four
+// fused multiply-adds (see gemm_f32.hip), so scores chained from channel 0 up and sums of values chained from the lowest key
+// up are the bits that block_partial gives.  A wave takes 16 queries, HW heads of a kv head for 16 / HW tokens on end, a
+// block four such waves; every block of 64 keys comes into LDS once for all of them, the next one on its way in registers
+// meanwhile.
+//   * scores S^T: first operand the keys, second the queries (in registers).  Row r of a tile of 16 keys is key
+//     4 (r % 4) + r / 4, so that a lane's results are keys 4 i + g of the tile (i = 0 .. 3, g = lane / 16): what step i of
+//     the products with the values takes from lane group g, so probabilities never move;
+//   * maxima and sums over the 64 keys: in the lane, then over the four lane groups.  The sum is wave_sum's tree, keys 32, 16,
+//     8, 4, 2, 1 apart, whose first four levels lie inside a lane;
+//   * O^T: first operand the values, 16 channels a tile.  Keys that a query does not see have probability zero and a chain
+//     goes on through zeros unchanged, unless such a key's value is not finite: a block that holds one takes the sums key
+//     by key, over the keys that a query sees.
+// Blocks whose tokens belong to several requests work off one request after the other.  What bounds it: a wave's own chain of
+// products, maxima, exponentials and sums, block after block (16 queries a wave are barely one wave a SIMD at the lengths of
+// ordinary prompts), a quarter of it MFMAs.  A prompt of 562 tokens, 32 heads of 64 on 8: 177 us multiplying one by one
+// (attention_tile_kernel), 60 us here; with the scores' bias looked at for every key 64 us, with the tokens' runs found one
+// token after the other 63 us.
+constexpr int kMfmaWaves = 4;
+
+template <int D, bool PLAIN>
+__global__ void __launch_bounds__(kMfmaWaves* kWave, D == 128 ? 1 : 2)
+attention_tile_mfma_kernel(const float* __restrict__ q, int q_stride, float* __restrict__ out, int out_stride, const float* __restrict__ k_pages,
+                           const float* __restrict__ v_pages, const int32_t* __restrict__ token_seq, const int32_t* __restrict__ positions,
+                           const int32_t* __restrict__ block_table, int bt_stride, int n_tokens, int n_q_heads, int n_kv_heads, int page_size,
+                           int page_shift, int window, float scale, int hw, float softcap, int chunk, const float* __restrict__ sinks,
+                           const float* __restrict__ slopes, const float* __restrict__ dist, int dist_len) {
+#pragma clang fp contract(off)
+  constexpr int kPitchK = D + 4, kPitchV = D;  // rows apart in banks as the operand reads want it
+  constexpr int kN = D / 16;                    // tiles of channels; row r of tile n is channel r * kN + n, so that a lane reads kN on end
+  constexpr int kRegionK = kWave * kPitchK > kMfmaWaves * kWave * 16 ? kWave * kPitchK : kMfmaWaves * kWave * 16;
+  constexpr int kPieces = 2 * D / 4;                 // 16-byte pieces of a key row and its value row
+  constexpr int kMoves = kWave * kPieces / (kMfmaWaves * kWave);
+  extern __shared__ __attribute__((aligned(16))) float tile_lds[];
+  float* k_t = tile_lds;
+  float* v_t = tile_lds + kRegionK;
+  __shared__ int not_finite[2];
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  const int n16 = lane % 16, g4 = lane / 16;
+  const int per_wave = 16 / hw, tokens = kMfmaWaves * per_wave;
+  const int t0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * tokens;  // the longest first
+  const int group = n_q_heads / n_kv_heads;
+  const int h = blockIdx.y * hw + n16 % hw, kvh = (blockIdx.y * hw) / group;
+  const int t_raw = t0 + wave * per_wave + n16 / hw;
+  const bool active = t_raw < n_tokens;
+  const int t = active ? t_raw : n_tokens - 1;
+  const int pos = positions[t];
+  const int seq = token_seq[t];
+  const int lo = first_key(pos, window, chunk);
+  const float slope = slopes ? slopes[h] : 0.f;
+  const float* my_dist = dist ? dist + (size_t)h * dist_len : nullptr;
+  float qs[D / 4];  // channels 4 s + g4 of this lane's query
+#pragma unroll
+  for (int s = 0; s < D / 4; ++s) qs[s] = q[(size_t)t * q_stride + (size_t)h * D + 4 * s + g4];
+  f32x4_t acc[D / 16];
+#pragma unroll
+  for (int c = 0; c < D / 16; ++c) acc[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  if (tid < 2) not_finite[tid] = 0;
+
+  const int count = min(tokens, n_tokens - t0);  // at most 64: a lane each
+  const int seq_of = lane < count ? token_seq[t0 + lane] : -1;
+  const int pos_of = lane < count ? positions[t0 + lane] : 0;
+  int turn = 0;  // which flag a pass uses
+  for (int first = 0; first < count;) {  // one request after the other
+    const int seq0 = __builtin_amdgcn_readlane(seq_of, first);
+    const unsigned long long others = __ballot(seq_of != seq0) >> first << first;
+    const int end = others ? min(__builtin_ctzll(others), count) : count;
+    const bool in_run = lane >= first && lane < end;
+    int key_lo = in_run ? first_key(pos_of, window, chunk) : INT_MAX, key_hi = in_run ? pos_of : -1;
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o /= 2) {
+      key_lo = min(key_lo, __shfl_xor(key_lo, o, kWave));
+      key_hi = max(key_hi, __shfl_xor(key_hi, o, kWave));
+    }
+    key_lo = __builtin_amdgcn_readfirstlane(key_lo);
+    key_hi = __builtin_amdgcn_readfirstlane(key_hi);
+    first = end;
+    const int32_t* bt = block_table + (size_t)seq0 * bt_stride;
+    const bool mine = seq == seq0;
+    f32x4_t held[kMoves];
+    unsigned seen = 0;  // bit u: somebody in the block sees the key of piece u, and its page is there (not given back by a window)
+    auto fetch = [&](int j0) {  // no branches: all pages are asked for together, then all pieces
+      int page[kMoves], in_page[kMoves];
+      auto key = [&](int u) { return min(max(j0 + (tid + u * kMfmaWaves * kWave) / kPieces, key_lo), key_hi); };
+      if (page_shift >= 0) {
+#pragma unroll
+        for (int u = 0; u < kMoves; ++u) page[u] = bt[key(u) >> page_shift], in_page[u] = key(u) & (page_size - 1);
+      } else {
+#pragma unroll
+        for (int u = 0; u < kMoves; ++u) page[u] = bt[key(u) / page_size], in_page[u] = key(u) % page_size;
+      }
+      seen = 0;
+#pragma unroll
+      for (int u = 0; u < kMoves; ++u) {
+        const int idx = tid + u * kMfmaWaves * kWave;
+        const int piece = idx % kPieces;
+        const bool is_k = piece < D / 4;
+        seen |= (key(u) == j0 + idx / kPieces && page[u] >= 0) ? 1u << u : 0u;
+        const size_t row = ((size_t)max(page[u], 0) * n_kv_heads + kvh) * page_size + (size_t)in_page[u];
+        held[u] = *reinterpret_cast<const f32x4_t*>((is_k ? k_pages : v_pages) + row * D + 4 * (is_k ? piece : piece - D / 4));
+      }
+    };
+    const int blk_lo = key_lo - key_lo % kWave;
+    fetch(blk_lo);
+    for (int j0 = blk_lo; j0 <= key_hi; j0 += kWave, turn ^= 1) {
+      __syncthreads();  // everybody has finished with the tiles of the block before
+      if (tid == 0) not_finite[turn ^ 1] = 0;  // (for the next pass: nobody reads or sets it now)
+      bool odd = false;
+#pragma unroll
+      for (int u = 0; u < kMoves; ++u) {
+        const int idx = tid + u * kMfmaWaves * kWave;
+        const int piece = idx % kPieces, r = idx / kPieces;
+        if (!(seen >> u & 1)) held[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        if (piece < D / 4) {
+          *reinterpret_cast<f32x4_t*>(k_t + r * kPitchK + 4 * piece) = held[u];
+        } else {
+          *reinterpret_cast<f32x4_t*>(v_t + r * kPitchV + 4 * (piece - D / 4)) = held[u];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) odd |= !(fabsf(held[u][e]) < INFINITY);
+        }
+      }
+      if (odd) not_finite[turn] = 1;
+      __syncthreads();
+      const bool by_key = not_finite[turn] != 0;
+      if (j0 + kWave <= key_hi) fetch(j0 + kWave);
+
+      f32x4_t c[4];
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) c[kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      const float* kr = k_t + (4 * (n16 % 4) + n16 / 4) * kPitchK + g4;
+      float ka[2][4][4];  // operands of 16 MFMAs, the next ones on their way meanwhile
+      auto read_keys = [&](int ch) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int kt = 0; kt < 4; ++kt) ka[ch % 2][s][kt] = kr[kt * 16 * kPitchK + 16 * ch + 4 * s];
+      };
+      read_keys(0);
+#pragma unroll
+      for (int ch = 0; ch < D / 16; ++ch) {
+        if (ch + 1 < D / 16) read_keys(ch + 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int kt = 0; kt < 4; ++kt) c[kt] = mfma_f32(ka[ch % 2][s][kt], qs[4 * ch + s], c[kt]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      const bool touched = mine & (j0 >= lo - lo % kWave) & (j0 <= pos);
+      float m_b = -INFINITY;
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int j = j0 + 16 * kt + 4 * i + g4;
+          const bool valid = mine & (j >= lo) & (j <= pos);
+          const float scaled = c[kt][i] * scale;
+          const float sc = PLAIN ? scaled : biased(capped(scaled, softcap), valid ? pos - j : 0, slope, my_dist, dist_len);
+          c[kt][i] = valid ? sc : -INFINITY;
+          m_b = fmaxf(m_b, c[kt][i]);
+        }
+      m_b = fmaxf(m_b, __shfl_xor(m_b, 16, kWave));
+      m_b = fmaxf(m_b, __shfl_xor(m_b, 32, kWave));
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int j = j0 + 16 * kt + 4 * i + g4;
+          const bool valid = mine & (j >= lo) & (j <= pos);
+          const float e = expf(c[kt][i] - m_b);
+          c[kt][i] = valid ? e : 0.f;
+        }
+      float half[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) half[i] = (c[0][i] + c[2][i]) + (c[1][i] + c[3][i]);
+      float l_b = (half[0] + half[2]) + (half[1] + half[3]);
+      l_b += __shfl_xor(l_b, 32, kWave);
+      l_b += __shfl_xor(l_b, 16, kWave);
+
+      f32x4_t o[D / 16];
+#pragma unroll
+      for (int n = 0; n < D / 16; ++n) o[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if (!by_key) {
+        const float* vr = v_t + g4 * kPitchV + n16 * kN;
+        float va[2][4][kN];
+        auto read_values = [&](int kt) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int n = 0; n < kN; ++n) va[kt % 2][i][n] = vr[(16 * kt + 4 * i) * kPitchV + n];
+        };
+        read_values(0);
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+          if (kt + 1 < 4) read_values(kt + 1);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int n = 0; n < kN; ++n) o[n] = mfma_f32(va[kt % 2][i][n], c[kt][i], o[n]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+        __syncthreads();  // the keys have been read: their place takes the probabilities, [wave][key][query]
+        float* p_t = k_t + wave * kWave * 16;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) p_t[(16 * kt + 4 * i + g4) * 16 + n16] = c[kt][i];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const int from = max(lo - j0, 0), to = touched ? min(pos - j0, kWave - 1) : -1;
+        for (int jj = from; jj <= to; ++jj)
+#pragma unroll
+          for (int n = 0; n < D / 16; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[n][i] = fmaf(p_t[jj * 16 + n16], v_t[jj * kPitchV + (4 * g4 + i) * kN + n], o[n][i]);
+      }
+      // the block joins the running result (merge_block), for the queries that see it
+      const float m_new = fmaxf(m, m_b);
+      const float keep = expf(m - m_new), take = expf(m_b - m_new);
+      l = touched ? fmaf(l, keep, l_b * take) : l;
+#pragma unroll
+      for (int n = 0; n < D / 16; ++n)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[n][i] = touched ? fmaf(acc[n][i], keep, o[n][i] * take) : acc[n][i];
+      m = touched ? m_new : m;
+    }
+  }
+  if (active) {
+    float* o = out + (size_t)t * out_stride + (size_t)h * D + 4 * g4 * kN;
+    const float inv_l = 1.0f / with_sink(l, m, sinks, h);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int n = 0; n < kN; ++n) o[i * kN + n] = acc[n][i] * inv_l;
+  }
+}
+
 // The same result from many waves, for steps with few tokens and long contexts (decode): wave
 // (token, head, r) computes block r of the token's key range alone and leaves it in `partials`
 // ([token][head][r][head_dim + 2]: the sums, then maximum and sum of probabilities); a second kernel
@@ -554,14 +795,15 @@ attention_join_kernel(T* __restrict__ out, int out_stride, const int32_t* __rest
 // pages: [page][n_kv_heads][page_size][head_dim].  token_seq[t]: row of block_table;
 // positions[t]: absolute position; the token sees positions max(0, p-window+1)..p (window 0: all).  slopes: one float
 // per query head (or null) that a capped score loses for every position between its key and the query; dist: a table
-// [n_q_heads][dist_len] (or null) of what it gains by distance instead.
+// [n_q_heads][dist_len] (or null) of what it gains by distance instead.  on_end: tokens stand in runs of many of one request
+// (prompts); the result is the same either way.
 TL_EXPORT int tl_attention_generic(const void* q, int q_stride, void* out, int out_stride,
                                    const void* k_pages, const void* v_pages, const int32_t* token_seq,
                                    const int32_t* positions, const int32_t* block_table, int bt_stride,
                                    int n_tokens, int n_q_heads, int n_kv_heads, int head_dim,
                                    int page_size, int window, float scale, float softcap, int chunk,
                                    const float* sinks, int v_dim, int v_pitch, int dtype, int keep_first, int n_v_heads,
-                                   const float* slopes, const float* dist, int dist_len, hipStream_t stream) {
+                                   const float* slopes, const float* dist, int dist_len, int on_end, hipStream_t stream) {
   TL_REQUIRE(n_tokens >= 0 && n_q_heads > 0 && n_kv_heads > 0 && page_size > 0 && bt_stride > 0,
              "attention: bad sizes");
   TL_REQUIRE(n_q_heads % n_kv_heads == 0, "attention: %d query heads are not a multiple of %d kv heads",
@@ -583,6 +825,45 @@ TL_EXPORT int tl_attention_generic(const void* q, int q_stride, void* out, int o
   const bool vec = head_dim % 4 == 0 && v_dim % 4 == 0 && v_pitch % 4 == 0 && ((uintptr_t)k_pages % 16) == 0 && ((uintptr_t)v_pages % 16) == 0;
   // prompt portions: tokens and heads that read the same keys share them through LDS (same bits)
   const size_t tile_lds = ((size_t)kTileWaves * head_dim + (size_t)kWave * (head_dim + v_dim + 2 * kTilePad)) * sizeof(float);
+  // ... in 32-bit on the matrix cores (a third of the time of the shared tiles, see there), if many tokens on end belong to a
+  // request (a block works off one request after the other, so that runs of one or two would wait for each other; whoever
+  // calls knows) and the sizes are those the kernel is built for
+  if (dtype == TL_F32 && on_end && n_tokens >= kTileMinTokens && vec && v_dim == head_dim && v_pitch == v_dim && n_v_heads == n_kv_heads &&
+      (keep_first == 0 || (window == 0 && chunk == 0)) && (head_dim == 16 || head_dim == 32 || head_dim == 64 || head_dim == 128)) {
+    const int group = n_q_heads / n_kv_heads;
+    const int hw = group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1);
+    const int tokens = kMfmaWaves * 16 / hw;
+    int page_shift = -1;
+    for (int sh = 0; sh < 31; ++sh)
+      if ((1 << sh) == page_size) page_shift = sh;
+    const dim3 mgrid((n_tokens + tokens - 1) / tokens, n_q_heads / hw);
+#define TL_MFMA_LAUNCH(D, PLAIN)                                                                                                        \
+  do {                                                                                                                               \
+    const int region_k = kWave * (D + 4) > kMfmaWaves * kWave * 16 ? kWave * (D + 4) : kMfmaWaves * kWave * 16;                      \
+    const int bytes = (region_k + kWave * D) * (int)sizeof(float);                                                                   \
+    if (bytes > 48 * 1024) {                                                                                                         \
+      hipError_t e = hipFuncSetAttribute((const void*)attention_tile_mfma_kernel<D, PLAIN>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes); \
+      if (e != hipSuccess) return tl_fail(TL_ERR_HIP, "attention: %s", hipGetErrorString(e));                                        \
+    }                                                                                                                                \
+    attention_tile_mfma_kernel<D, PLAIN><<<mgrid, kMfmaWaves * kWave, bytes, stream>>>(                                                     \
+        (const float*)q, q_stride, (float*)out, out_stride, (const float*)k_pages, (const float*)v_pages, token_seq, positions,      \
+        block_table, bt_stride, n_tokens, n_q_heads, n_kv_heads, page_size, page_shift, window, scale, hw, softcap, chunk, sinks,    \
+        slopes, dist, dist_len);                                                                                                     \
+  } while (0)
+    const bool plain = !(softcap > 0.f) && !slopes && !dist;
+#define TL_MFMA_EITHER(D)                       \
+  do {                                          \
+    if (plain) TL_MFMA_LAUNCH(D, true);         \
+    else TL_MFMA_LAUNCH(D, false);              \
+  } while (0)
+    if (head_dim == 16) TL_MFMA_EITHER(16);
+    else if (head_dim == 32) TL_MFMA_EITHER(32);
+    else if (head_dim == 64) TL_MFMA_EITHER(64);
+    else TL_MFMA_EITHER(128);
+#undef TL_MFMA_EITHER
+#undef TL_MFMA_LAUNCH
+    return tl_check_launch("attention_tile_mfma");
+  }
   if (n_tokens >= kTileMinTokens && tile_lds <= (size_t)tl_device_facts().lds_bytes) {  // (heads too large for the tiles walk alone: the same bits)
     const int group = n_q_heads / n_kv_heads;
     const int hb = group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1);

@@ -13,6 +13,9 @@ from . import ops
 
 #: contexts beyond this many keys give every block of 64 keys a wave of its own in the plain kernel
 GENERIC_SPLIT_FROM = 128
+#: prompt portions of this many tokens each on average count as runs on end for the plain kernel: a block of its 32-bit form
+#: for the matrix cores takes 16 tokens or more, one request after the other
+GENERIC_ON_END = 16
 
 
 def paged_attention(
@@ -132,6 +135,7 @@ def paged_attention(
         else:
             ops.attention_generic(
                 qkv[n_dec:], n_q_heads, n_kv_heads, head_dim, k_pages, v_pages, ctx.token_seq[n_dec:],
-                ctx.positions[n_dec:], ctx.block_tables[group], window, scale, out=out[n_dec:], **extras,
+                ctx.positions[n_dec:], ctx.block_tables[group], window, scale, out=out[n_dec:],
+                on_end=n - n_dec >= GENERIC_ON_END * (ctx.host.n_seqs - n_dec), **extras,
             )
     return out

@@ -111,6 +111,7 @@ def attention_generic(
     value_heads: Optional[int] = None,
     slopes: Optional[torch.Tensor] = None,
     distances: Optional[torch.Tensor] = None,
+    on_end: bool = False,
 ) -> torch.Tensor:
     """Attention of each token's query heads (the first Hq * dh columns of ``qkv``) over the paged
     keys and values of its request; returns [n, Hq * dv].  ``softcap`` c > 0: scores become
@@ -122,7 +123,8 @@ def attention_generic(
     the value pages have fewer heads than the key pages, and key head g reads value head ``g % value_heads``
     (several score maps over the same values: the key heads of map m are ``m * value_heads ..``).  ``slopes``: a bias by
     distance, one 32-bit number per query head that the capped score loses for every position between key and query.
-    ``distances`` float32 [Hq, entries], in place of slopes: what the capped score gains by distance, by table."""
+    ``distances`` float32 [Hq, entries], in place of slopes: what the capped score gains by distance, by table.  ``on_end``: the tokens stand in runs of
+    many of one request (which kernel is used; the result is the same)."""
     n, page_size, out, v_dim, v_pitch = _generic_arguments(qkv, n_q_heads, n_kv_heads, head_dim, k_pages, v_pages, token_seq,
                                                            positions, block_table, out, sinks, v_head_dim, values_in_keys, value_offset,
                                                            keep_first, value_heads)
@@ -132,7 +134,7 @@ def attention_generic(
             qkv.data_ptr(), qkv.stride(0), out.data_ptr(), out.stride(0), k_pages.data_ptr(), v_at,
             token_seq.data_ptr(), positions.data_ptr(), block_table.data_ptr(), block_table.stride(0), n,
             n_q_heads, n_kv_heads, head_dim, page_size, window, float(scale), float(softcap), int(chunk), _ptr(sinks), v_dim,
-            v_pitch, dtype_code(qkv.dtype), int(keep_first), int(value_heads or 0), _slopes(slopes, n_q_heads), *_distances(distances, n_q_heads), _stream(),
+            v_pitch, dtype_code(qkv.dtype), int(keep_first), int(value_heads or 0), _slopes(slopes, n_q_heads), *_distances(distances, n_q_heads), int(on_end), _stream(),
         )
     )
     return out
