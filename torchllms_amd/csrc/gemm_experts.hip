@@ -18,7 +18,7 @@
 //   * Blocks go to the eight XCDs in turn.  All row tiles of one (expert, column tile) go to the same XCD one after the
 //     other, so W is read from memory once and met again in that XCD's L2; an expert's column tiles are spread over all XCDs.
 // 8 experts of 4,096 x 3,584, gated + plain product: 16 pairs 119 us (a wave per 16 columns with operands straight from memory,
-// before: 156; the bytes of W at 6.1 TB/s: 101), 128 pairs 134 (235; 116), 4,096 pairs 518 (a library product per expert, with
+// before: 156; the bytes of W at 6.1 TB/s: 101), 128 pairs 123 (235; 116), 4,096 pairs 518 (a library product per expert, with
 // the activation in a kernel of its own: 632, and the host waited for the offsets once a layer) = 697 TFLOP/s.
 #include "common.h"
 
@@ -159,15 +159,22 @@ expert_tile_kernel(const bf16_t* __restrict__ rows, const bf16_t* __restrict__ w
   // all loads are unconditional (past the end the last step is fetched again and never used), so that a wave's count of
   // outstanding loads is the same in every trip
   const int steps = K / kStepE;
+  // rows of W lie a power of two apart, so blocks that walk K in step would all press on the same memory channels at once:
+  // the column tiles start their walks at different steps and wrap around (the row tiles of one at the same step: they share
+  // W in L2, and a row's sums do not depend on where it lies).  Eight experts of 2,048 x 2,048, 48 pairs: gated + plain product
+  // 35 + 18.8 us in step, 27.3 + 16.0 like this; of 4,096 x 3,584 90 + 42 and 80.5 + 42; 256 pairs 36.6 + 21.5 and 28.9 + 20.2.
+  // With 64 rows a tile it changes nothing, with 128 blocks lose what they share of the rows (4,096 pairs 299 + 150, and 328 + 159)
+  const int rot = BM <= 32 ? (n_tile * 5 + e * 3) % steps : 0;
+  auto step_of = [&](int i) { return i + rot < steps ? i + rot : i + rot - steps; };
 #pragma unroll
-  for (int s = 0; s < kStages - 1; ++s) issue(min(s, steps - 1), s);
+  for (int s = 0; s < kStages - 1; ++s) issue(step_of(min(s, steps - 1)), s);
   __builtin_amdgcn_s_waitcnt(S::kWait);
   __syncthreads();
   operands(0, 0);
   int buffer = 0;
   for (int i = 0; i < steps; ++i) {
     // (everybody passed the barrier below after reading the last of step i - 1, whose buffer is filled again here)
-    issue(min(i + kStages - 1, steps - 1), buffer == 0 ? kStages - 1 : buffer - 1);
+    issue(step_of(min(i + kStages - 1, steps - 1)), buffer == 0 ? kStages - 1 : buffer - 1);
     operands(buffer, 1);
     __builtin_amdgcn_sched_barrier(0);
     multiply(0);
