@@ -643,6 +643,46 @@ def test_attention_generic_on_the_matrix_cores_gives_the_same_bits(hq, hkv, dh, 
     assert torch.equal(want.nan_to_num(7.0), got.nan_to_num(7.0))
 
 
+@pytest.mark.parametrize("n, outputs, K", [(1, 1, 8), (3, 16, 520), (256, 9, 2048), (257, 9, 2048), (5, 17, 4096), (24, 10, 4104)])
+def test_routing_in_one_launch_or_two(n, outputs, K):
+    """The router's product and the choice, at the edges of what one launch takes (256 tokens, 16 outputs, a gate's column
+    behind the outputs that are chosen from), against 64 bits: sums of K products, each rounded once at most.  The choice is
+    the one that the kernel for given outputs makes."""
+    ops = _ops()
+    torch.manual_seed(n + K)
+    x, w = torch.randn(n, K).bfloat16(), torch.randn(outputs, K).bfloat16()
+    n_out = max(outputs - 1, 1)
+    top = min(2, n_out)
+    bias = torch.randn(n_out, device=DEV)
+    z, ids, weights = ops.route(x.to(DEV), w.to(DEV), n_out, None, top, bias=bias, normalize=True)
+    bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    assert bool(((z.cpu().double() - x.double() @ w.double().t()).abs() <= bound).all())
+    want_ids, want_weights = ops.router_topk(z, n_out, None, top, bias=bias, normalize=True)
+    assert torch.equal(ids, want_ids) and torch.equal(weights, want_weights)
+
+
+@pytest.mark.parametrize("n, top, D", [(1, 1, 8), (64, 2, 520), (43, 3, 64), (65, 2, 20)])
+@pytest.mark.parametrize("weighed", [False, True])
+def test_pairs_are_gathered_in_one_launch_or_two(n, top, D, weighed):
+    """128 pairs and one more, outputs that nobody chose, widths that are no multiple of a load: every pair's row is its
+    token's, and an output's rows lie between its offsets."""
+    ops, n_out = _ops(), 7
+    torch.manual_seed(n)
+    x, ids = torch.randn(n, D).bfloat16(), torch.randint(1, n_out - 1, (n, top), dtype=torch.int32)
+    weights = torch.rand(n, top) if weighed else None
+    rows, pos, offsets = ops.expert_gather(x.to(DEV), ids.to(DEV), n_out, input_weights=weights.to(DEV) if weighed else None)
+    assert offsets.tolist() == [int((ids < e).sum()) for e in range(n_out + 1)]
+    at = pos.cpu().flatten().long()
+    assert sorted(at.tolist()) == list(range(n * top))
+    flat = ids.flatten().long()
+    start = offsets.cpu().long()
+    assert bool(((at >= start[flat]) & (at < start[flat + 1])).all())
+    want = x.repeat_interleave(top, 0)
+    if weighed:
+        want = (weights.flatten()[:, None] * want.float()).bfloat16()
+    assert torch.equal(rows.cpu()[at], want)
+
+
 def test_attention_window_never_reads_released_pages():
     """Blocks wholly before the window are -1 in the block table; the kernel must not touch them."""
     torch.manual_seed(0)

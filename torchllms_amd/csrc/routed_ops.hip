@@ -1,6 +1,8 @@
 // Kernels of a routed feed-forward (a mixture of experts whose router's scores are a softmax, with a correction
 // added for the choice only, and whose last outputs may be experts that hand their input through), of dense
 // feed-forwards (biases and the exact gelu; the squared relu), and of layers with a norm on either side of every branch.
+#include <limits.h>
+
 #include "common.h"
 
 namespace {
@@ -17,14 +19,24 @@ __device__ __forceinline__ float sigmoid_r(float z) { return 1.0f / (1.0f + expf
 // logistic function of every z by itself instead of the softmax over all (without a correction the largest z are chosen,
 // which are the largest s also where these round to the same number).
 constexpr int kRouterPerLane = 8;  // outputs a lane holds: up to 512 experts
-__global__ void __launch_bounds__(256)
-router_topk_kernel(const float* __restrict__ z, int z_stride, const float* __restrict__ correction, int n, int n_out, int top,
-                   int32_t* __restrict__ ids, float* __restrict__ weights, int n_groups, int keep_groups, int normalize,
-                   float route_scale, const float* __restrict__ bias, int sigmoid) {
-  const int t = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
-  const int lane = threadIdx.x % kWave;
-  if (t >= n) return;
-  const float* zr = z + (size_t)t * z_stride;
+struct Choice {
+  const float* correction;
+  int n_out, top;
+  int32_t* ids;
+  float* weights;
+  int n_groups, keep_groups, normalize;
+  float route_scale;
+  const float* bias;
+  int sigmoid;
+};
+
+// One wave: token t, its row of router outputs zr (memory or LDS).
+__device__ __forceinline__ void choose(const float* zr, int t, int lane, const Choice& a) {
+  const float *correction = a.correction, *bias = a.bias;
+  const int n_out = a.n_out, top = a.top, n_groups = a.n_groups, keep_groups = a.keep_groups, normalize = a.normalize, sigmoid = a.sigmoid;
+  const float route_scale = a.route_scale;
+  int32_t* ids = a.ids;
+  float* weights = a.weights;
   float s[kRouterPerLane], c[kRouterPerLane];
   float mx = -INFINITY;
 #pragma unroll
@@ -109,6 +121,55 @@ router_topk_kernel(const float* __restrict__ z, int z_stride, const float* __res
     for (int k = 0; k < top; ++k) total += w[k];
     for (int k = 0; k < top; ++k) w[k] = (normalize ? w[k] / (total + 1e-20f) : w[k]) * route_scale;
   }
+}
+
+__global__ void __launch_bounds__(256) router_topk_kernel(const float* __restrict__ z, int z_stride, int n, const Choice a) {
+  const int t = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+  if (t < n) choose(z + (size_t)t * z_stride, t, threadIdx.x % kWave, a);
+}
+
+// The router's product and the choice in one launch, for steps of few tokens (bfloat16 rows and matrix, widths in eights):
+// a block a token, a wave an output, a lane eight neighbouring elements a round with the loads of
+// eight rounds in flight; the first wave chooses.  z [n, rows] is stored too (columns from n_out on are other gates').  What
+// bounds it: launch and latency; the matrix comes from L2 once a token.  In a replayed graph, nine outputs, product by
+// gemm_stream or gemm_wide and choice in launches of their own | one: width 2,048, 1 token 6.7 | 6.0 us, 24 tokens 9.5 | 6.4, 256
+// tokens 9.8 | 6.6; width 4,096 7.6 | 6.1, 10.3 | 6.6, 10.5 | 6.9.  (A wave for several outputs, one after the other: 33 outputs
+// 8.0 | 9.9 with one token of 4,096, 64 outputs 8.4 | 14.1, hence a wave for one.)
+constexpr int kRouterThreads = 1024;
+constexpr int kRouterFewRows = kRouterThreads / kWave;  // outputs: a wave each
+typedef __bf16 bf16x8_z __attribute__((ext_vector_type(8)));
+__global__ void __launch_bounds__(kRouterThreads)
+router_product_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, int K, int rows, float* __restrict__ z, const Choice a) {
+  __shared__ float z_l[kRouterFewRows];
+  const int t = blockIdx.x, wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const bf16_t* xr = x + (size_t)t * K;
+  if (wave < rows) {
+    const int o = wave;
+    const bf16_t* wr = w + (size_t)o * K;
+    float sum = 0.f;
+    constexpr int kAhead = 8;
+    for (int k0 = 0; k0 < K; k0 += kAhead * kWave * 8) {
+      bf16x8_z xv[kAhead], wv[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int k = k0 + (u * kWave + lane) * 8;
+        xv[u] = *reinterpret_cast<const bf16x8_z*>(xr + (k < K ? k : 0));
+        wv[u] = *reinterpret_cast<const bf16x8_z*>(wr + (k < K ? k : 0));
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u)
+        if (k0 + (u * kWave + lane) * 8 < K)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) sum = fmaf((float)xv[u][i], (float)wv[u][i], sum);
+    }
+    sum = wave_sum(sum);
+    if (lane == 0) {
+      z_l[o] = sum;
+      z[(size_t)t * rows + o] = sum;
+    }
+  }
+  __syncthreads();
+  if (wave == 0) choose(z_l, t, lane, a);
 }
 
 // ----------------------------------------------------------------------------- experts over their gathered rows
@@ -432,6 +493,49 @@ expert_gather_kernel(const T* __restrict__ x, const float* __restrict__ weights,
   }
 }
 
+// Places and copies in one launch, for steps of few pairs: every block counts for itself how many pairs lie before its own
+// (those of lower outputs, and earlier ones of the same), and one block more writes the offsets.
+// Width 2,048 in a replayed graph: 48 pairs 5.0 us in two launches, 2.6 in one; at 256 pairs 5.0 and 5.6 (counting grows).
+constexpr int kGatherPairs = 128;  // a pair a thread
+template <typename T, int V>
+__global__ void __launch_bounds__(kGatherPairs)
+expert_place_gather_kernel(const T* __restrict__ x, const float* __restrict__ weights, const int32_t* __restrict__ ids, int pairs, int top, int n_out,
+                           int32_t* __restrict__ offsets, int32_t* __restrict__ pos, T* __restrict__ rows, int D) {
+  __shared__ int id_l[kGatherPairs];
+  __shared__ int before[kGatherPairs / kWave];
+  const int tid = threadIdx.x, p = blockIdx.x;
+  const int id = tid < pairs ? ids[tid] : INT_MAX;
+  if (p == pairs) {
+    id_l[tid] = id;
+    __syncthreads();
+    for (int e = tid; e <= n_out; e += kGatherPairs) {
+      int sum = 0;
+      for (int q = 0; q < pairs; ++q) sum += id_l[q] < e;
+      offsets[e] = sum;
+    }
+    return;
+  }
+  const int mine = ids[p];
+  const int count = __popcll(__ballot(id < mine || (id == mine && tid < p)));
+  if (tid % kWave == 0) before[tid / kWave] = count;
+  __syncthreads();
+  int at = 0;
+#pragma unroll
+  for (int u = 0; u < kGatherPairs / kWave; ++u) at += before[u];
+  if (tid == 0) pos[p] = at;
+  struct alignas(sizeof(T) * V) Vec { T e[V]; };
+  const T* src = x + (size_t)(p / top) * D;
+  T* dst = rows + (size_t)at * D;
+  const float w = weights ? weights[p] : 1.f;
+  for (int d = tid * V; d < D; d += kGatherPairs * V) {
+    Vec v = *reinterpret_cast<const Vec*>(src + d);
+    if (weights)
+#pragma unroll
+      for (int e = 0; e < V; ++e) v.e[e] = from_f32<T>(w * to_f32(v.e[e]));
+    *reinterpret_cast<Vec*>(dst + d) = v;
+  }
+}
+
 // out[p, d] = T(weights[p] * x[p / top, d]): the pairs' inputs in their own order.
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -726,19 +830,26 @@ __global__ void __launch_bounds__(256) relu_square_kernel(T* __restrict__ x, siz
 }  // namespace
 
 // ============================================================================= C interface
-TL_EXPORT int tl_router_topk(const float* z, int z_stride, const float* correction, int n, int n_out, int top, int32_t* ids,
+// x != null: z [n, z_stride] is worked out here, x [n, K] times w [z_stride, K] (bfloat16), otherwise it is given.
+TL_EXPORT int tl_router_topk(float* z, int z_stride, const float* correction, int n, int n_out, int top, int32_t* ids,
                              float* weights, int n_groups, int keep_groups, int normalize, float route_scale, const float* bias,
-                             int sigmoid, hipStream_t stream) {
+                             int sigmoid, const void* x, const void* w, int K, hipStream_t stream) {
   TL_REQUIRE(n >= 0 && n_out > 0 && top > 0 && top <= n_out && z_stride >= n_out, "router_topk: bad sizes");
   TL_REQUIRE(n_groups >= 0 && (n_groups == 0 || (n_groups <= kWave && n_out % n_groups == 0 && keep_groups > 0 && keep_groups <= n_groups
                                                  && (long long)keep_groups * (n_out / n_groups) >= top)),
              "router_topk: %d groups of which %d stay do not fit %d outputs and %d choices (at most 64 groups)", n_groups, keep_groups, n_out, top);
   if (n_out > kRouterPerLane * kWave)
     return tl_fail(TL_ERR_UNSUPPORTED, "router_topk: %d router outputs, at most %d", n_out, kRouterPerLane * kWave);
+  TL_REQUIRE(!x || (w && K > 0 && K % 8 == 0 && z_stride <= kRouterFewRows && ((uintptr_t)x | (uintptr_t)w) % 16 == 0),
+             "router_topk: the product here takes widths in eights, aligned rows and up to %d outputs", kRouterFewRows);
   if (n == 0) return TL_OK;
   const int per_block = 256 / kWave;
-  router_topk_kernel<<<(n + per_block - 1) / per_block, 256, 0, stream>>>(z, z_stride, correction, n, n_out, top, ids, weights, n_groups,
-                                                                         keep_groups, normalize, route_scale, bias, sigmoid);
+  const Choice choice = {correction, n_out, top, ids, weights, n_groups, keep_groups, normalize, route_scale, bias, sigmoid};
+  if (x) {
+    router_product_kernel<<<n, kRouterThreads, 0, stream>>>((const bf16_t*)x, (const bf16_t*)w, K, z_stride, z, choice);
+    return tl_check_launch("router_product");
+  }
+  router_topk_kernel<<<(n + per_block - 1) / per_block, 256, 0, stream>>>(z, z_stride, n, choice);
   return tl_check_launch("router_topk");
 }
 
@@ -834,10 +945,16 @@ TL_EXPORT int tl_expert_gather(const void* x, const int32_t* ids, const float* w
   if (n == 0) return TL_OK;
   if (dtype != TL_F32 && dtype != TL_BF16) return tl_fail(TL_ERR_ARG, "expert_gather: unknown dtype %d", dtype);
   const int pairs = n * top;
-  expert_places_kernel<<<1, kPlaceThreads, 0, stream>>>(ids, pairs, n_out, offsets, pos);
+  const bool few = pairs <= kGatherPairs;  // (beyond, every block's count of all pairs is the longer way)
+  if (!few) expert_places_kernel<<<1, kPlaceThreads, 0, stream>>>(ids, pairs, n_out, offsets, pos);
   const int vec = dtype == TL_F32 ? 4 : 8;  // elements of 16 bytes
   const bool wide = D % vec == 0 && ((uintptr_t)x | (uintptr_t)rows) % 16 == 0;
-#define TL_GATHER(T, V) expert_gather_kernel<T, V><<<pairs, 256, 0, stream>>>((const T*)x, weights, top, pos, (T*)rows, D)
+#define TL_GATHER(T, V)                                                                                                             \
+  do {                                                                                                                              \
+    if (few) expert_place_gather_kernel<T, V><<<pairs + 1, kGatherPairs, 0, stream>>>((const T*)x, weights, ids, pairs, top, n_out, \
+                                                                                      offsets, pos, (T*)rows, D);                   \
+    else expert_gather_kernel<T, V><<<pairs, 256, 0, stream>>>((const T*)x, weights, top, pos, (T*)rows, D);                        \
+  } while (0)
   if (dtype == TL_F32) {
     if (wide) TL_GATHER(float, 4);
     else TL_GATHER(float, 1);

@@ -139,6 +139,7 @@ from .routed_ops import (  # noqa: F401
     pair_norm_add_norm,
     post_norm_add_norm,
     relu_square_,
+    route,
     router_topk,
     weighted_pair,
 )

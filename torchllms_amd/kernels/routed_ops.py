@@ -10,15 +10,32 @@ from typing import Optional, Tuple
 import torch
 
 from .base import F32, KernelError, _gpu, _ptr, _stream, check, core, dtype_code
+from .products import linear
 
 #: the most outputs a router may have (experts and experts that hand their input through together)
 ROUTER_MAX_OUTPUTS = 512
 ROUTER_SCORES = {"softmax": 0, "sigmoid": 1}
+#: the most outputs and tokens that ``route`` multiplies and chooses in one launch
+ROUTE_OUTPUTS, ROUTE_TOKENS = 16, 256
+
+
+def route(x: torch.Tensor, w_router: torch.Tensor, n_out: int, correction: Optional[torch.Tensor], top: int, **options):
+    """``router_topk`` of ``z = x w_router^T`` (32-bit).  Returns ``(z, ids, weights)``.  Steps of few tokens of bfloat16
+    models are one launch if a block has a wave for every output."""
+    _gpu(x, w_router)
+    rows, K = w_router.shape
+    if not (x.dtype == torch.bfloat16 == w_router.dtype and x.dim() == 2 and x.shape[1] == K and 0 < x.shape[0] <= ROUTE_TOKENS
+            and rows <= ROUTE_OUTPUTS and K % 8 == 0 and x.is_contiguous() and w_router.is_contiguous()
+            and (x.data_ptr() | w_router.data_ptr()) % 16 == 0):
+        z = linear(x, w_router, out_dtype=torch.float32)
+        return (z,) + router_topk(z, n_out, correction, top, **options)
+    z = torch.empty((x.shape[0], rows), dtype=torch.float32, device=x.device)
+    return (z,) + router_topk(z, n_out, correction, top, product=(x, w_router), **options)
 
 
 def router_topk(z: torch.Tensor, n_out: int, correction: Optional[torch.Tensor], top: int, groups: int = 0, keep_groups: int = 0,
                 normalize: bool = False, scale: float = 1.0, bias: Optional[torch.Tensor] = None,
-                scores: str = "softmax") -> Tuple[torch.Tensor, torch.Tensor]:
+                scores: str = "softmax", product: Optional[Tuple[torch.Tensor, torch.Tensor]] = None) -> Tuple[torch.Tensor, torch.Tensor]:
     """``z`` float32 [n, >= n_out]: the router's outputs in the first ``n_out`` columns.  ``s = softmax(z)``; the
     ``top`` outputs with the largest ``s + correction`` are chosen (of equal ones the lower index).  Returns
     ``(ids int32 [n, top], weights float32 [n, top])``, the weights being the chosen outputs' ``s``.  ``correction``
@@ -27,7 +44,7 @@ def router_topk(z: torch.Tensor, n_out: int, correction: Optional[torch.Tensor],
     are divided by their sum (+ 1e-20); ``scale`` then multiplies them.  ``bias`` (float32 [n_out]) is added to ``z``
     first; with ``normalize`` the weights are then the softmax of ``z + bias`` over the chosen outputs alone.
     ``scores`` "sigmoid": ``s`` is the logistic function of every output by itself instead of the softmax over all (without
-    a correction the choice is the largest outputs', also where their ``s`` round to one number)."""
+    a correction the choice is the largest outputs', also where their ``s`` round to one number).  ``product`` (x, w): ``z``, contiguous, is written first (``route`` says when)."""
     if scores not in ROUTER_SCORES:
         raise KernelError(f"router_topk: scores {scores!r} ({sorted(ROUTER_SCORES)})")
     _gpu(z, correction, bias)
@@ -44,7 +61,8 @@ def router_topk(z: torch.Tensor, n_out: int, correction: Optional[torch.Tensor],
     ids = torch.empty((n, top), dtype=torch.int32, device=z.device)
     weights = torch.empty((n, top), dtype=torch.float32, device=z.device)
     check(core().tl_router_topk(z.data_ptr(), z.stride(0), _ptr(correction), n, n_out, top, ids.data_ptr(), weights.data_ptr(),
-                                int(groups), int(keep_groups), 1 if normalize else 0, float(scale), _ptr(bias), ROUTER_SCORES[scores], _stream()))
+                                int(groups), int(keep_groups), 1 if normalize else 0, float(scale), _ptr(bias), ROUTER_SCORES[scores],
+                                _ptr(product[0] if product else None), _ptr(product[1] if product else None), product[0].shape[1] if product else 0, _stream()))
     return ids, weights
 
 

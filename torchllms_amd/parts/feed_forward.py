@@ -207,9 +207,8 @@ class RoutedExperts(FeedForward):
     def forward(self, x, ctx):
         x = ops.resolved(x)
         n_out = self.E + self.I
-        z = ops.linear(x, self.w_router, out_dtype=torch.float32)
-        ids, weights = ops.router_topk(z, n_out, self.correction, self.top, groups=self.groups, keep_groups=self.keep_groups,
-                                       normalize=self.normalize, scale=self.route_scale, bias=self.router_bias, scores=self.scores)
+        z, ids, weights = ops.route(x, self.w_router, n_out, self.correction, self.top, groups=self.groups, keep_groups=self.keep_groups,
+                                    normalize=self.normalize, scale=self.route_scale, bias=self.router_bias, scores=self.scores)
         inputs = None  # weights of the experts' inputs; the results are then added as they are
         if self.weigh_input:
             inputs, weights = weights, None
