@@ -40,6 +40,13 @@ def test_short_uneven_requests_in_numbers_are_left_whole():
         assert ops.decode_splits(*args) == ops.plan_decode_splits(*args)
 
 
+def test_requests_of_512_keys_and_fewer_are_left_whole_from_half_a_pair_a_cu_on():
+    for head_dim in (32, 64, 128):
+        assert ops.decode_splits(16, 8, 512, head_dim) == ops.decode_splits(128, 1, 100, head_dim, uneven=True) == (512, 1)
+    for args in ((16, 8, 513, 64), (15, 8, 512, 128), (16, 8, 512, 256)):  # longer, fewer, or wider heads: as planned
+        assert ops.decode_splits(*args) == ops.plan_decode_splits(*args)
+
+
 def test_a_sampled_row_is_cut_only_when_rows_are_few_and_long():
     assert ops.sample_chunks(1, 128256) == 15 and ops.sample_chunks(8, 128256) == 15
     assert ops.sample_chunks(64, 128256) == 4 and ops.sample_chunks(256, 128256) == 1
