@@ -388,10 +388,11 @@ def test_layernorm_of_every_width(hidden, stream, out):
 # ----------------------------------------------------------------------------- routed experts' products by tiles
 @pytest.mark.parametrize("counts, D, F", [
     ([1], 64, 64), ([0, 3, 0, 17, 1, 0], 128, 192), ([15, 16, 17, 33], 64, 320), ([31, 0, 32, 65], 192, 64), ([64, 63, 129, 0, 65], 128, 448),
-    ([127, 128, 129], 64, 192), ([300, 1, 0, 520], 320, 128), ([513], 64, 64), ([2, 0, 1] * 30, 64, 128), ([0, 0, 40] * 44, 64, 64)])
+    ([127, 128, 129], 64, 192), ([300, 1, 0, 520], 320, 128), ([513], 64, 64), ([2, 0, 1] * 30, 64, 128), ([0, 0, 40] * 44, 64, 64),
+    ([600, 1, 255], 64, 5184), ([600, 1, 255], 10304, 64)])
 def test_expert_products_by_tiles(counts, D, F):
     """Every tile size (chosen by the mean rows of an expert), experts without rows, one row, a tile's edge, columns that
-    are no multiple of a tile, one step along K, more experts than a wave has lanes, and rows behind the last expert's
+    are no multiple of a tile (with the large tiles of either product among them), one step along K, more experts than a wave has lanes, and rows behind the last expert's
     (pairs of outputs that are no experts), which stay unwritten."""
     ops = _ops()
     g = torch.Generator().manual_seed(sum(counts) + D)

@@ -13,13 +13,15 @@
 //   * GLU: a wave's rows of W are half gate rows, half up rows of the same columns, so the gate meets its up product in
 //     registers.
 //   * Tiles by the rows an expert has on average: 128 x 128 for prompts (bound by LDS reads and the matrix cores, which take
-//     about the same time; two blocks a CU fill each other's gaps), 16, 32 or 64 rows for decode steps and short prompts
+//     about the same time; two blocks a CU fill each other's gaps) and 128 x 256 for long ones (below), 16, 32 or 64 rows for decode steps and short prompts
 //     (bound by reading W: many blocks with several steps in flight).
 //   * Blocks go to the eight XCDs in turn.  All row tiles of one (expert, column tile) go to the same XCD one after the
 //     other, so W is read from memory once and met again in that XCD's L2; an expert's column tiles are spread over all XCDs.
 // 8 experts of 4,096 x 3,584, gated + plain product: 16 pairs 119 us (a wave per 16 columns with operands straight from memory,
 // before: 156; the bytes of W at 6.1 TB/s: 101), 128 pairs 123 (235; 116), 4,096 pairs 518 (a library product per expert, with
-// the activation in a kernel of its own: 632, and the host waited for the offsets once a layer) = 697 TFLOP/s.
+// the activation in a kernel of its own: 632, and the host waited for the offsets once a layer), 408 by the large tiles.
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -59,19 +61,11 @@ struct ExpertTile {
   static constexpr int kWait = (kPending & 0xF) | (0x7 << 4) | (0xF << 8) | ((kPending >> 4) << 14);
 };
 
-template <int BM, int BN, int WAVES_M, int kStages, bool GLU>
-__global__ void __launch_bounds__(256)
-expert_tile_kernel(const bf16_t* __restrict__ rows, const bf16_t* __restrict__ w, const int32_t* __restrict__ offsets, int n_experts,
-                   bf16_t* __restrict__ mid, float* __restrict__ y, int K, int N) {
-  using S = ExpertTile<BM, BN, WAVES_M, kStages, GLU>;
-  constexpr int MT = S::MT, NT = S::NT;
-  extern __shared__ __attribute__((aligned(16))) bf16_t lds_e[];
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int n16 = lane % 16, g4 = lane / 16;
-
-  // which tile: XCD x walks, expert after expert, its column tiles n = x, x + 8, ... (the start shifted from expert to
-  // expert, so that a number of tiles that is no multiple of 8 evens out), the row tiles of each side by side
-  const int n_tiles = (N + S::kColumns - 1) / S::kColumns;
+// Which tile a block takes: XCD x walks, expert after expert, its column tiles n = x, x + 8, ... (the start shifted from expert
+// to expert, so that a number of tiles that is no multiple of 8 evens out), the row tiles of each side by side.  False: none.
+struct Tile { int e, n_tile, r0, hi; };
+template <int BM>
+__device__ __forceinline__ bool find_tile(const int32_t* __restrict__ offsets, int n_experts, int n_tiles, int lane, Tile& t) {
   const int per_xcd = (n_tiles + kXcds - 1) / kXcds;
   const int x = blockIdx.x % kXcds;
   int j = blockIdx.x / kXcds;  // place among this XCD's tiles
@@ -94,12 +88,28 @@ expert_tile_kernel(const bf16_t* __restrict__ rows, const bf16_t* __restrict__ w
     }
     j -= __shfl(sum, kWave - 1, kWave) * per_xcd;
   }
-  if (e < 0) return;
-  e = __builtin_amdgcn_readfirstlane(e);
-  const int n_tile = __builtin_amdgcn_readfirstlane((j / m_tiles) * kXcds + (x + e * (n_tiles % kXcds)) % kXcds);
-  if (n_tile >= n_tiles) return;
-  const int hi = offsets[e + 1];
-  const int r0 = __builtin_amdgcn_readfirstlane(offsets[e] + (j % m_tiles) * BM);
+  if (e < 0) return false;
+  t.e = __builtin_amdgcn_readfirstlane(e);
+  t.n_tile = __builtin_amdgcn_readfirstlane((j / m_tiles) * kXcds + (x + t.e * (n_tiles % kXcds)) % kXcds);
+  if (t.n_tile >= n_tiles) return false;
+  t.hi = offsets[t.e + 1];
+  t.r0 = __builtin_amdgcn_readfirstlane(offsets[t.e] + (j % m_tiles) * BM);
+  return true;
+}
+
+template <int BM, int BN, int WAVES_M, int kStages, bool GLU>
+__global__ void __launch_bounds__(256)
+expert_tile_kernel(const bf16_t* __restrict__ rows, const bf16_t* __restrict__ w, const int32_t* __restrict__ offsets, int n_experts,
+                   bf16_t* __restrict__ mid, float* __restrict__ y, int K, int N) {
+  using S = ExpertTile<BM, BN, WAVES_M, kStages, GLU>;
+  constexpr int MT = S::MT, NT = S::NT;
+  extern __shared__ __attribute__((aligned(16))) bf16_t lds_e[];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int n16 = lane % 16, g4 = lane / 16;
+
+  Tile tile;
+  if (!find_tile<BM>(offsets, n_experts, (N + S::kColumns - 1) / S::kColumns, lane, tile)) return;
+  const int e = tile.e, n_tile = tile.n_tile, r0 = tile.r0, hi = tile.hi;
   const int n0 = n_tile * S::kColumns;
   const bf16_t* we = w + (size_t)e * (GLU ? 2 : 1) * N * K;
 
@@ -162,9 +172,9 @@ expert_tile_kernel(const bf16_t* __restrict__ rows, const bf16_t* __restrict__ w
   // rows of W lie a power of two apart, so blocks that walk K in step would all press on the same memory channels at once:
   // the column tiles start their walks at different steps and wrap around (the row tiles of one at the same step: they share
   // W in L2, and a row's sums do not depend on where it lies).  Eight experts of 2,048 x 2,048, 48 pairs: gated + plain product
-  // 35 + 18.8 us in step, 27.3 + 16.0 like this; of 4,096 x 3,584 90 + 42 and 80.5 + 42; 256 pairs 36.6 + 21.5 and 28.9 + 20.2.
-  // With 64 rows a tile it changes nothing, with 128 blocks lose what they share of the rows (4,096 pairs 299 + 150, and 328 + 159)
-  const int rot = BM <= 32 ? (n_tile * 5 + e * 3) % steps : 0;
+  // 35 + 18.8 us in step, 27.3 + 16.0 like this; of 4,096 x 3,584 90 + 42 and 80.5 + 42; 256 pairs 36.6 + 21.5 and 28.9 + 20.2 (94 + 54 and 88 + 55).
+  // With 128 rows a tile blocks lose what they share of the rows (4,096 pairs 299 + 150, and 328 + 159)
+  const int rot = BM <= 64 ? (n_tile * 5 + e * 3) % steps : 0;
   auto step_of = [&](int i) { return i + rot < steps ? i + rot : i + rot - steps; };
 #pragma unroll
   for (int s = 0; s < kStages - 1; ++s) issue(step_of(min(s, steps - 1)), s);
@@ -234,6 +244,144 @@ int launch_expert_tiles(const void* rows, const void* w, const int32_t* offsets,
   return tl_check_launch("expert_tiles");
 }
 
+// The same with 128 x 256 tiles, for prompts: a wave takes 64 x 128 of it, so that it reads three quarters of the LDS bytes an
+// MFMA that 64 x 64 reads.  K in steps of 32 (64 bytes a row, piece p at slot p ^ (r / 2 % 4)), three buffers of 24 KB, so that
+// two blocks share a CU; a step's operands are read while the step before is multiplied, one barrier a step.
+constexpr int kWideM = 128, kWideN = 256, kWideStep = 32, kWideStage = (kWideM + kWideN) * kWideStep;  // (elements)
+template <bool GLU>
+__global__ void __launch_bounds__(256, 2)
+expert_wide_tile_kernel(const bf16_t* __restrict__ rows, const bf16_t* __restrict__ w, const int32_t* __restrict__ offsets, int n_experts,
+                        bf16_t* __restrict__ mid, float* __restrict__ y, int K, int N) {
+  constexpr int kColumns = GLU ? kWideN / 2 : kWideN, WM = 64, WN = 128, MT = WM / 16, NT = WN / 16, kLoads = 6;
+  extern __shared__ __attribute__((aligned(16))) bf16_t lds_e[];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int n16 = lane % 16, g4 = lane / 16;
+  Tile tile;
+  if (!find_tile<kWideM>(offsets, n_experts, (N + kColumns - 1) / kColumns, lane, tile)) return;
+  const int e = tile.e, r0 = tile.r0, hi = tile.hi;
+  const int n0 = tile.n_tile * kColumns;
+  const bf16_t* we = w + (size_t)e * (GLU ? 2 : 1) * N * K;
+
+  // instruction j of the wave fills 16 rows of the buffer: two of rows, four of W
+  const int r16 = lane / 4, piece = 8 * ((lane % 4) ^ (r16 / 2 % 4));
+  const bf16_t* src[kLoads];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) src[j] = rows + (size_t)min(r0 + (wave * 2 + j) * 16 + r16, hi - 1) * K + piece;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int r = (wave * 4 + j) * 16 + r16;
+    int row;
+    if constexpr (GLU) {
+      const int in = r % WN, half = in / (WN / 2);
+      row = half * N + min(n0 + (r / WN) * (WN / 2) + in % (WN / 2), N - 1);
+    } else {
+      row = min(n0 + r, N - 1);
+    }
+    src[2 + j] = we + (size_t)row * K + piece;
+  }
+  const uint32_t base = (uint32_t)(uintptr_t)lds_e;
+  const uint32_t a_at = __builtin_amdgcn_readfirstlane(base + wave * 2 * 1024);
+  const uint32_t w_at = __builtin_amdgcn_readfirstlane(base + kWideM * kWideStep * 2 + wave * 4 * 1024);
+  auto issue = [&](int step, int buffer) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) rows_to_lds(src[j] + step * kWideStep, a_at + buffer * kWideStage * 2 + j * 1024);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) rows_to_lds(src[2 + j] + step * kWideStep, w_at + buffer * kWideStage * 2 + j * 1024);
+  };
+  float4_e acc[NT][MT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int c = 0; c < MT; ++c) acc[t][c] = float4_e{0.f, 0.f, 0.f, 0.f};
+  const int am = (wave % 2) * WM, wn = wave / 2;
+  const int at = n16 * kWideStep + 8 * (g4 ^ (n16 / 2 % 4));
+  bf16x8_e wop[2][NT], aop[2][MT];
+  auto operands = [&](auto set, int buffer) {
+    const bf16_t* as = lds_e + buffer * kWideStage + am * kWideStep + at;
+    const bf16_t* ws = lds_e + buffer * kWideStage + (kWideM + wn * WN) * kWideStep + at;
+#pragma unroll
+    for (int c = 0; c < MT; ++c) aop[set][c] = *reinterpret_cast<const bf16x8_e*>(as + c * 16 * kWideStep);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) wop[set][t] = *reinterpret_cast<const bf16x8_e*>(ws + t * 16 * kWideStep);
+  };
+  auto multiply = [&](auto set) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int c = 0; c < MT; ++c) acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wop[set][t], aop[set][c], acc[t][c], 0, 0, 0);
+  };
+  // s_waitcnt: loads of all but the `steps` latest steps have landed; LDS reads too where `lds` is 0
+  constexpr auto wait = [](int steps, int lds) { return (steps * kLoads & 0xF) | (0x7 << 4) | (lds << 8) | (steps * kLoads >> 4 << 14); };
+  const int steps = K / kWideStep;  // (even: K is a multiple of 64)
+  int b = 0;                        // buffer of step i
+  // (loads are unconditional, as above)
+  auto pass = [&](int i, auto set, auto next) {
+    // this wave's operands of step i are in registers and its loads of step i + 1 in LDS; after the barrier everybody's are, and
+    // the buffer of step i is free
+    __builtin_amdgcn_s_waitcnt(wait(1, 0));
+    __syncthreads();
+    issue(min(i + 3, steps - 1), b);
+    b = b == 2 ? 0 : b + 1;
+    operands(next, b);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(set);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  using Zero = std::integral_constant<int, 0>;
+  using One = std::integral_constant<int, 1>;
+#pragma unroll
+  for (int s = 0; s < 3; ++s) issue(min(s, steps - 1), s);
+  __builtin_amdgcn_s_waitcnt(wait(2, 0xF));
+  __syncthreads();
+  operands(Zero(), 0);
+  for (int i = 0; i < steps; i += 2) {
+    pass(i, Zero(), One());
+    pass(i + 1, One(), Zero());
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // the last, unused fetches must not land after the block has gone
+
+  // acc[t][c][i]: row r0 + am + 16 c + n16, W row 16 t + 4 g4 + i of the wave's
+#pragma unroll
+  for (int c = 0; c < MT; ++c) {
+    const int r = r0 + am + 16 * c + n16;
+    if (r >= hi) continue;
+    if constexpr (GLU) {
+#pragma unroll
+      for (int t = 0; t < NT / 2; ++t) {
+        const int n = n0 + wn * (WN / 2) + 16 * t + 4 * g4;
+        if (n >= N) continue;  // (N is a multiple of 4)
+        bf16x4_e out;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float g = acc[t][c][i];
+          out[i] = (__bf16)(g / (1.0f + expf(-g)) * acc[t + NT / 2][c][i]);
+        }
+        *reinterpret_cast<bf16x4_e*>(mid + (size_t)r * N + n) = out;
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const int n = n0 + wn * WN + 16 * t + 4 * g4;
+        if (n < N) *reinterpret_cast<float4_e*>(y + (size_t)r * N + n) = acc[t][c];
+      }
+    }
+  }
+}
+
+template <bool GLU>
+int launch_expert_wide(const void* rows, const void* w, const int32_t* offsets, int n_experts, void* mid, float* y, int K, int N, int pairs,
+                       hipStream_t stream) {
+  constexpr int kLds = 3 * kWideStage * 2, kColumns = GLU ? kWideN / 2 : kWideN;
+  const auto kernel = expert_wide_tile_kernel<GLU>;
+  hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+  if (err != hipSuccess) return tl_fail(TL_ERR_HIP, "expert products: %s", hipGetErrorString(err));
+  const int per_xcd = ((N + kColumns - 1) / kColumns + kXcds - 1) / kXcds;
+  const int most = (pairs < n_experts ? pairs : n_experts) + pairs / kWideM;  // row tiles there can be
+  kernel<<<dim3((unsigned)(kXcds * per_xcd) * most), 256, kLds, stream>>>((const bf16_t*)rows, (const bf16_t*)w, offsets, n_experts, (bf16_t*)mid, y,
+                                                                        K, N);
+  return tl_check_launch("expert_wide_tiles");
+}
+
 }  // namespace
 
 // Sizes the kernel takes: K a multiple of a step, columns in fours.
@@ -244,11 +392,18 @@ bool tl_expert_tiles_fit(int K, int N) { return K % kStepE == 0 && N % 4 == 0; }
 // Which tile: by the rows an expert has on average (`pairs` counts those of outputs that are no experts too).  Measured at
 // 8 experts, gated + plain product in us, widths 4,096 x 3,584 | 2,048 x 2,048, with 16, 32, 64 and 128 rows a tile:
 // 16 pairs 119 120 119 - | 48 48 54 -; 256 pairs (32 rows) 163 137 135 173 | 61 59 55 79; 1,024 pairs (128 rows) - - 227 235
-// | - - 84 87; 2,424 pairs (303 rows) - - 371 364 | - - 127 125; 4,096 pairs - - 592 518 | - - 195 195.  (128 x 256 tiles
-// with one block a CU: 585 at 4,096 pairs.)
+// | - - 84 87; 2,424 pairs (303 rows) - - 371 364 | - - 127 125; 4,096 pairs - - 592 518 | - - 195 195.  128 x 256 tiles where
+// they are more than five for four CUs, 128 x 128 and 128 x 256: 2,424 pairs 234 + 137 and 223 + 132, 4,096 pairs 308 + 147 and
+// 265 + 143; where they are fewer the CUs that get none weigh more (2,048 x 2,048, 288 of them for the plain product: 47 and 50;
+// 4,096 x 1,024 gated, 288: 82 and 87).  (128 x 256 tiles with K in steps of 64 and one block a CU: 585 at 4,096 pairs.)
 int tl_expert_tiles(const void* rows, const void* w, const int32_t* offsets, int n_experts, void* mid, float* y, int K, int N, int pairs,
                     hipStream_t stream) {
   const double mean = (double)pairs / n_experts;
+  // (the large tiles there will be, every expert's last one half empty)
+  const double large = (pairs / (double)kWideM + 0.5 * n_experts) * ((N + (mid ? kWideN / 2 : kWideN) - 1) / (mid ? kWideN / 2 : kWideN));
+  if (mean > 256 && large > 1.25 * tl_device_facts().compute_units)
+    return mid ? launch_expert_wide<true>(rows, w, offsets, n_experts, mid, y, K, N, pairs, stream)
+               : launch_expert_wide<false>(rows, w, offsets, n_experts, mid, y, K, N, pairs, stream);
 #define TL_TILES(BM, BN, WM, ST, GLU) return launch_expert_tiles<BM, BN, WM, ST, GLU>(rows, w, offsets, n_experts, mid, y, K, N, pairs, stream)
   if (mid) {
     if (mean <= 12) TL_TILES(16, 128, 1, 4, true);
