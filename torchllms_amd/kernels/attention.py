@@ -14,8 +14,10 @@ from . import ops
 #: contexts beyond this many keys give every block of 64 keys a wave of its own in the plain kernel
 GENERIC_SPLIT_FROM = 128
 #: prompt portions of this many tokens each on average count as runs on end for the plain kernel: a block of its 32-bit form
-#: for the matrix cores takes 16 tokens or more, one request after the other
-GENERIC_ON_END = 16
+#: for the matrix cores takes 16 tokens or more, one request after the other.  256 tokens of 32 heads of 64 behind 64 | 512 |
+#: 2,048 keys, us, shared tiles and matrix cores: portions of 4 tokens 30 and 43 | 140 and 170 | 570 and 609, of 8 tokens 32 and
+#: 25 | 142 and 89 | 531 and 306, of 16 31 and 18 | 142 and 48 | 516 and 156; heads of 128 cross at the same place.
+GENERIC_ON_END = 8
 
 
 def paged_attention(
