@@ -415,6 +415,42 @@ def test_expert_products_by_tiles(counts, D, F):
         assert bool(((y[at].double() - x @ w.T).abs() <= F * 2.0 ** -24 * (x.abs() @ w.abs().T) + 1e-30).all())
 
 
+@pytest.mark.parametrize("tokens, E, D, F, prompt", [(256, 8, 256, 192, True), (600, 4, 320, 128, True), (1030, 3, 64, 5184, True),
+                                                     (255, 8, 256, 192, True), (600, 4, 320, 128, False)])
+def test_routed_experts_of_prompts_round_as_dense_layers(tokens, E, D, F, prompt):
+    """A bfloat16 step with prompts and at least 512 pairs gives what the dense layers' products give expert by expert (the
+    gate, the up product and the activation rounded to bfloat16 on the way), with tiles of 64, 128 and 128 x 256; fewer pairs
+    and decode steps round the gated product once."""
+    from types import SimpleNamespace
+
+    from torchllms_amd.parts.feed_forward import RoutedExperts
+
+    ops = _ops()
+    g = torch.Generator().manual_seed(tokens + D)
+    part = RoutedExperts(D, F, E, 2, correction=False)
+    tensors = {n: (torch.randn(s.shape, generator=g) * (0.5 if "router" in n else 0.1)).bfloat16().to(DEV) for n, s in part.param_specs().items()}
+    part.bind(tensors)
+    x = torch.randn(tokens, D, generator=g).bfloat16().to(DEV)
+    got = part.forward(x, SimpleNamespace(host=SimpleNamespace(max_q_len=tokens if prompt else 1)))
+    _, ids, weights = ops.route(x, part.w_router, E, None, 2)
+    rows, pos, offsets = ops.expert_gather(x, ids, E)
+    y = torch.empty(2 * tokens, D, device=DEV)
+    apart = torch.empty_like(y)
+    for e in range(E):
+        at = slice(int(offsets[e]), int(offsets[e + 1]))
+        y[at] = ops.linear(ops.silu_mul(ops.linear(rows[at], part.w_gu[e])), part.w_down[e], out_dtype=torch.float32)
+        both = ops.linear(rows[at], part.w_gu[e], out_dtype=torch.float32)
+        apart[at] = ops.linear((torch.nn.functional.silu(both[:, :F]) * both[:, F:]).bfloat16(), part.w_down[e], out_dtype=torch.float32)
+    dense, once = (ops.expert_combine(r, pos, ids, weights, E, x) for r in (y, apart))
+    # sums in another order (K roundings to 24 bits, which add up like sqrt(K)) cross a rounding to 8 bits at a share of about
+    # sqrt(K) / 2^15 of the entries, at three roundings before the second product and one behind; a dropped rounding moves
+    # every second result
+    share = lambda a, b: (a != b).float().mean().item()  # noqa: E731
+    like_dense = prompt and 2 * tokens >= 512
+    near, far = (dense, once) if like_dense else (once, dense)
+    assert share(got, near) <= 4 * max(D, F) ** 0.5 / 2 ** 15 + 0.005 and share(got, far) > 0.1, (share(got, near), share(got, far))
+
+
 # ----------------------------------------------------------------------------- attention
 def _paged(k, v, page, n_pages, seed=0, dtype=torch.float32):
     """Scatter dense per-request keys/values [S, Hkv, dh] into shuffled pages; returns pages and

@@ -1,6 +1,6 @@
 // The products of routed experts over their gathered rows, bfloat16 inputs, 32-bit sums: for every expert e,
 // C[r, n] = rows[r] . W[e][n] for its rows offsets[e] .. offsets[e + 1], or (GLU) mid[r, n] = silu(rows[r] . Wgate[e][n]) *
-// (rows[r] . Wup[e][n]), rounded once.  How many rows an expert got is known on the device only, so one launch covers all
+// (rows[r] . Wup[e][n]), rounded once or as dense layers round (gated, below).  How many rows an expert got is known on the device only, so one launch covers all
 // experts: a block finds its tile from the offsets, and blocks beyond the last tile end at once.  Nothing is read back, and
 // the launch depends on the step's shape alone (it can be recorded).
 //
@@ -43,6 +43,19 @@ __device__ __forceinline__ void rows_to_lds(const bf16_t* src, uint32_t lds_at) 
       :
       : "v"(src), "s"(lds_at)
       : "m0", "memory");
+}
+
+// silu(gate) * up of four columns.  rounded: the two products and the activation are rounded to bfloat16 on the way, as dense
+// layers' are (silu_mul of a product stored in bfloat16); otherwise the result alone is.
+__device__ __forceinline__ bf16x4_e gated(const float4_e& gate, const float4_e& up, bool rounded) {
+  bf16x4_e out;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float g = rounded ? (float)(__bf16)gate[i] : gate[i], u = rounded ? (float)(__bf16)up[i] : up[i];
+    const float act = g / (1.0f + expf(-g));
+    out[i] = (__bf16)((rounded ? (float)(__bf16)act : act) * u);
+  }
+  return out;
 }
 
 template <int BM, int BN, int WAVES_M, int kStages, bool GLU>
@@ -100,7 +113,7 @@ __device__ __forceinline__ bool find_tile(const int32_t* __restrict__ offsets, i
 template <int BM, int BN, int WAVES_M, int kStages, bool GLU>
 __global__ void __launch_bounds__(256)
 expert_tile_kernel(const bf16_t* __restrict__ rows, const bf16_t* __restrict__ w, const int32_t* __restrict__ offsets, int n_experts,
-                   bf16_t* __restrict__ mid, float* __restrict__ y, int K, int N) {
+                   bf16_t* __restrict__ mid, float* __restrict__ y, int K, int N, bool rounded) {
   using S = ExpertTile<BM, BN, WAVES_M, kStages, GLU>;
   constexpr int MT = S::MT, NT = S::NT;
   extern __shared__ __attribute__((aligned(16))) bf16_t lds_e[];
@@ -209,13 +222,7 @@ expert_tile_kernel(const bf16_t* __restrict__ rows, const bf16_t* __restrict__ w
       for (int t = 0; t < NT / 2; ++t) {
         const int n = n0 + wn * (S::WN / 2) + 16 * t + 4 * g4;
         if (n >= N) continue;  // (N is a multiple of 4)
-        bf16x4_e out;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float g = acc[t][c][i];
-          out[i] = (__bf16)(g / (1.0f + expf(-g)) * acc[t + NT / 2][c][i]);
-        }
-        *reinterpret_cast<bf16x4_e*>(mid + (size_t)r * N + n) = out;
+        *reinterpret_cast<bf16x4_e*>(mid + (size_t)r * N + n) = gated(acc[t][c], acc[t + NT / 2][c], rounded);
       }
     } else {
 #pragma unroll
@@ -229,7 +236,7 @@ expert_tile_kernel(const bf16_t* __restrict__ rows, const bf16_t* __restrict__ w
 
 template <int BM, int BN, int WAVES_M, int kStages, bool GLU>
 int launch_expert_tiles(const void* rows, const void* w, const int32_t* offsets, int n_experts, void* mid, float* y, int K, int N, int pairs,
-                        hipStream_t stream) {
+                        bool rounded, hipStream_t stream) {
   using S = ExpertTile<BM, BN, WAVES_M, kStages, GLU>;
   const auto kernel = expert_tile_kernel<BM, BN, WAVES_M, kStages, GLU>;
   if (S::kLdsBytes > 48 * 1024) {
@@ -240,7 +247,7 @@ int launch_expert_tiles(const void* rows, const void* w, const int32_t* offsets,
   const int per_xcd = (n_tiles + kXcds - 1) / kXcds;
   const int most = (pairs < n_experts ? pairs : n_experts) + pairs / BM;  // row tiles there can be
   kernel<<<dim3((unsigned)(kXcds * per_xcd) * most), 256, S::kLdsBytes, stream>>>((const bf16_t*)rows, (const bf16_t*)w, offsets, n_experts,
-                                                                               (bf16_t*)mid, y, K, N);
+                                                                               (bf16_t*)mid, y, K, N, rounded);
   return tl_check_launch("expert_tiles");
 }
 
@@ -251,7 +258,7 @@ constexpr int kWideM = 128, kWideN = 256, kWideStep = 32, kWideStage = (kWideM +
 template <bool GLU>
 __global__ void __launch_bounds__(256, 2)
 expert_wide_tile_kernel(const bf16_t* __restrict__ rows, const bf16_t* __restrict__ w, const int32_t* __restrict__ offsets, int n_experts,
-                        bf16_t* __restrict__ mid, float* __restrict__ y, int K, int N) {
+                        bf16_t* __restrict__ mid, float* __restrict__ y, int K, int N, bool rounded) {
   constexpr int kColumns = GLU ? kWideN / 2 : kWideN, WM = 64, WN = 128, MT = WM / 16, NT = WN / 16, kLoads = 6;
   extern __shared__ __attribute__((aligned(16))) bf16_t lds_e[];
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
@@ -350,13 +357,7 @@ expert_wide_tile_kernel(const bf16_t* __restrict__ rows, const bf16_t* __restric
       for (int t = 0; t < NT / 2; ++t) {
         const int n = n0 + wn * (WN / 2) + 16 * t + 4 * g4;
         if (n >= N) continue;  // (N is a multiple of 4)
-        bf16x4_e out;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float g = acc[t][c][i];
-          out[i] = (__bf16)(g / (1.0f + expf(-g)) * acc[t + NT / 2][c][i]);
-        }
-        *reinterpret_cast<bf16x4_e*>(mid + (size_t)r * N + n) = out;
+        *reinterpret_cast<bf16x4_e*>(mid + (size_t)r * N + n) = gated(acc[t][c], acc[t + NT / 2][c], rounded);
       }
     } else {
 #pragma unroll
@@ -370,7 +371,7 @@ expert_wide_tile_kernel(const bf16_t* __restrict__ rows, const bf16_t* __restric
 
 template <bool GLU>
 int launch_expert_wide(const void* rows, const void* w, const int32_t* offsets, int n_experts, void* mid, float* y, int K, int N, int pairs,
-                       hipStream_t stream) {
+                       bool rounded, hipStream_t stream) {
   constexpr int kLds = 3 * kWideStage * 2, kColumns = GLU ? kWideN / 2 : kWideN;
   const auto kernel = expert_wide_tile_kernel<GLU>;
   hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
@@ -378,7 +379,7 @@ int launch_expert_wide(const void* rows, const void* w, const int32_t* offsets, 
   const int per_xcd = ((N + kColumns - 1) / kColumns + kXcds - 1) / kXcds;
   const int most = (pairs < n_experts ? pairs : n_experts) + pairs / kWideM;  // row tiles there can be
   kernel<<<dim3((unsigned)(kXcds * per_xcd) * most), 256, kLds, stream>>>((const bf16_t*)rows, (const bf16_t*)w, offsets, n_experts, (bf16_t*)mid, y,
-                                                                        K, N);
+                                                                        K, N, rounded);
   return tl_check_launch("expert_wide_tiles");
 }
 
@@ -387,7 +388,8 @@ int launch_expert_wide(const void* rows, const void* w, const int32_t* offsets, 
 // Sizes the kernel takes: K a multiple of a step, columns in fours.
 bool tl_expert_tiles_fit(int K, int N) { return K % kStepE == 0 && N % 4 == 0; }
 
-// mid != null: the gated product (w [E, 2 N, K], gate rows then up rows), otherwise y = the plain one (w [E, N, K]).
+// mid != null: the gated product (w [E, 2 N, K], gate rows then up rows; rounded: as dense layers do), otherwise y = the plain one
+// (w [E, N, K]).
 //
 // Which tile: by the rows an expert has on average (`pairs` counts those of outputs that are no experts too).  Measured at
 // 8 experts, gated + plain product in us, widths 4,096 x 3,584 | 2,048 x 2,048, with 16, 32, 64 and 128 rows a tile:
@@ -397,14 +399,14 @@ bool tl_expert_tiles_fit(int K, int N) { return K % kStepE == 0 && N % 4 == 0; }
 // 265 + 143; where they are fewer the CUs that get none weigh more (2,048 x 2,048, 288 of them for the plain product: 47 and 50;
 // 4,096 x 1,024 gated, 288: 82 and 87).  (128 x 256 tiles with K in steps of 64 and one block a CU: 585 at 4,096 pairs.)
 int tl_expert_tiles(const void* rows, const void* w, const int32_t* offsets, int n_experts, void* mid, float* y, int K, int N, int pairs,
-                    hipStream_t stream) {
+                    bool rounded, hipStream_t stream) {
   const double mean = (double)pairs / n_experts;
   // (the large tiles there will be, every expert's last one half empty)
   const double large = (pairs / (double)kWideM + 0.5 * n_experts) * ((N + (mid ? kWideN / 2 : kWideN) - 1) / (mid ? kWideN / 2 : kWideN));
   if (mean > 256 && large > 1.25 * tl_device_facts().compute_units)
-    return mid ? launch_expert_wide<true>(rows, w, offsets, n_experts, mid, y, K, N, pairs, stream)
-               : launch_expert_wide<false>(rows, w, offsets, n_experts, mid, y, K, N, pairs, stream);
-#define TL_TILES(BM, BN, WM, ST, GLU) return launch_expert_tiles<BM, BN, WM, ST, GLU>(rows, w, offsets, n_experts, mid, y, K, N, pairs, stream)
+    return mid ? launch_expert_wide<true>(rows, w, offsets, n_experts, mid, y, K, N, pairs, rounded, stream)
+               : launch_expert_wide<false>(rows, w, offsets, n_experts, mid, y, K, N, pairs, rounded, stream);
+#define TL_TILES(BM, BN, WM, ST, GLU) return launch_expert_tiles<BM, BN, WM, ST, GLU>(rows, w, offsets, n_experts, mid, y, K, N, pairs, rounded, stream)
   if (mid) {
     if (mean <= 12) TL_TILES(16, 128, 1, 4, true);
     if (mean <= 24) TL_TILES(32, 128, 1, 4, true);

@@ -46,7 +46,7 @@ _CORE_SIGNATURES = {
     "tl_streams_update": [_P, _I, _I64, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P],
     "tl_streams_open": [_P, _P, _I, _I64, _P],
     "tl_maps_join": [_P, _I, _P, _I, _I, _I, _F, _F, _F, _I, _P],
-    "tl_expert_glu_rows": [_P, _P, _P, _I, _P, _I, _I, _I, _I, _P],
+    "tl_expert_glu_rows": [_P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _P],
     "tl_expert_down_rows": [_P, _P, _P, _I, _P, _I, _I, _I, _I, _P],
     "tl_expert_gather": [_P, _P, _P, _I, _I, _I, _P, _P, _P, _I, _I, _P],
     "tl_pair_rows": [_P, _P, _P, _I, _I, _I, _I, _P],

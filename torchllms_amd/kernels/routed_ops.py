@@ -89,11 +89,13 @@ def expert_tiles_fit(width: int, expert_size: int) -> bool:
     return width % 64 == 0 and expert_size % 64 == 0
 
 
-def expert_glu_rows(rows: torch.Tensor, w_gate_up: torch.Tensor, offsets: torch.Tensor) -> torch.Tensor:
+def expert_glu_rows(rows: torch.Tensor, w_gate_up: torch.Tensor, offsets: torch.Tensor, rounded: bool = False) -> torch.Tensor:
     """``mid[r] = silu(Wg[e] rows[r]) * (Wu[e] rows[r])`` for the rows ``offsets[e] .. offsets[e + 1]`` of every expert
     ``e`` of ``w_gate_up`` [E, 2F, D] (gate rows, then up rows); ``rows`` [pairs, D] as ``expert_gather`` leaves them.
     An expert's weights are read once for a tile of its rows.  Returns [pairs, F]; rows behind ``offsets[E]`` (pairs of
-    outputs that are no experts) are left unwritten."""
+    outputs that are no experts) are left unwritten.  ``rounded`` (bfloat16, ``expert_tiles_fit``): the two products and the
+    activation are rounded to bfloat16 on the way, as ``silu_mul(linear(..))`` and so dense layers round; otherwise the result
+    alone is."""
     _gpu(rows, w_gate_up, offsets)
     _expert_rows(rows, w_gate_up, offsets, "expert_glu_rows")
     if w_gate_up.shape[1] % 2:
@@ -101,7 +103,7 @@ def expert_glu_rows(rows: torch.Tensor, w_gate_up: torch.Tensor, offsets: torch.
     E, F, D = w_gate_up.shape[0], w_gate_up.shape[1] // 2, rows.shape[1]
     mid = torch.empty((rows.shape[0], F), dtype=rows.dtype, device=rows.device)
     check(core().tl_expert_glu_rows(rows.data_ptr(), w_gate_up.data_ptr(), offsets.data_ptr(), E, mid.data_ptr(), D, F,
-                                    rows.shape[0], dtype_code(rows.dtype), _stream()))
+                                    rows.shape[0], dtype_code(rows.dtype), 1 if rounded else 0, _stream()))
     return mid
 
 
