@@ -174,3 +174,55 @@ def test_matrix_memory_by_chunks(lengths, H, dk, dv):
     for s in states:
         top = s[:, H * (dv + 1) * dk : H * (dv + 1) * (dk + 1)].view(len(lengths), H, dv + 1).double()
         assert bool(((top - tops[..., None]).abs() <= 1e-5 * (1 + tops[..., None].abs())).all())
+
+
+@pytest.mark.parametrize("what", ["q", "k", "v"])
+@pytest.mark.parametrize("rule", ["head", "channel", "plain", "memory"])
+def test_a_token_that_is_not_finite_spoils_no_earlier_one(rule, what):
+    """An infinity in a query, key or value at the start, in the middle and at the end of a chunk, of one head of one request:
+    earlier tokens, the other head and the other requests keep their bits; from it on, and in the states, the same places
+    are finite as in the token-by-token walk."""
+    from torchllms_amd.kernels import ops
+
+    H, dk, dv, lengths = 2, 64, 24, [1, 40, 50, 17]
+    offsets = torch.tensor([0] + lengths).cumsum(0).int()
+    n, rows = int(offsets[-1]), len(lengths)
+    g = torch.Generator().manual_seed(7)
+    qk, vw = H * dk, H * dv
+    data = torch.randn((n, 2 * qk + 2 * vw + 2 * H), generator=g).bfloat16()  # queries, keys, values, gate, two gates a head
+    a = torch.randn((n, H * dk), generator=g) - 4.0
+    A_log, bias, norm_w = torch.rand(H, generator=g), torch.randn(H * dk, generator=g) * 0.5, torch.rand(vw, generator=g) + 0.5
+    per = ops.matrix_memory_state_size(H, dk, dv) if rule == "memory" else H * dv * dk
+    start = torch.randn((rows, per + -per % 4), generator=g)
+    if rule == "memory":
+        start.zero_()
+    where = (offsets.to(DEV), torch.arange(rows, dtype=torch.int32, device=DEV))
+
+    def run(x, longest):
+        state, x = start.to(DEV), x.to(DEV)
+        kw = dict(longest=longest, single_rows=1)
+        if rule == "memory":
+            out = ops.matrix_memory(x, 0, qk, 2 * qk, 2 * qk + 2 * vw, 2 * qk + 2 * vw + H, 2 * qk + vw, bias[:H].to(DEV), bias[H : 2 * H].to(DEV),
+                                    9.0, norm_w.to(DEV), EPS, state, 0, *where, H, dk, dv, **kw)
+        elif rule == "plain":
+            out = ops.gated_linear(x[:, : 2 * qk + vw], a.to(DEV), bias.to(DEV), 0.25, x, 2 * qk + vw, norm_w[:dv].to(DEV), EPS, state, 0, *where, H, dk, dv, **kw)
+        else:
+            out = ops.gated_delta(x[:, : 2 * qk + vw], x, 2 * qk + vw, 2 * qk + 2 * vw, 2 * qk + 2 * vw + H, A_log.to(DEV),
+                                  (bias if rule == "channel" else bias[:H]).to(DEV), norm_w[:dv].to(DEV), EPS, state, 0, *where, H, H, dk, dv,
+                                  channel_decay=a.to(DEV) if rule == "channel" else None, **kw)
+        return out.cpu().float(), state.cpu()
+
+    clean, clean_state = run(data, max(lengths))
+    assert bool(torch.isfinite(clean).all())
+    for place in (16, 21, 31, 39):  # of the second row, tokens 1 .. 40
+        at = 1 + place
+        x = data.clone()
+        x[at, {"q": 0, "k": qk, "v": 2 * qk}[what] + 5] = float("inf")  # of head 0
+        out, state = run(x, max(lengths))
+        walked, walked_state = run(x, 0)
+        spoiled = torch.zeros(n, vw, dtype=torch.bool)
+        spoiled[at : at + 1 if what == "q" else 41, :dv] = True
+        assert torch.equal(out[~spoiled], clean[~spoiled])
+        assert torch.equal(torch.isfinite(out), torch.isfinite(walked)) and not bool(torch.isfinite(out[at, :dv]).all())
+        assert torch.equal(torch.isfinite(state), torch.isfinite(walked_state))
+        assert torch.equal(state[[0, 2, 3]], clean_state[[0, 2, 3]])

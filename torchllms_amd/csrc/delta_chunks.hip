@@ -16,7 +16,9 @@
 //     rows of S as accumulators of its MFMAs, whose layout is that of the operand of the products with S (step i of an
 //     MFMA takes rows 4 g + i), so S never leaves its registers; the waves' parts of Kt S and Qt S meet in LDS behind the
 //     one barrier of a chunk, then every wave forms u for itself, again operand for operand in registers.  A chunk's
-//     operands are asked for two chunks ahead.
+//     operands are asked for two chunks ahead.  A chunk with values that are not finite takes its two triangular products row
+//     by row (causal_product): a token's infinity reaches itself and later ones alone, as in the walk.  (The look at every
+//     chunk's values costs the delta rules 1 to 2%: 2,048 tokens 240 -> 242 us in all, 4 x 3,000 1,532 -> 1,561.)
 // What bounds it: the walk, a chain of one chunk behind the other (about 0.6 us each: 16 + 4 + 8 MFMAs of 32 cycles and a
 // barrier): a prompt of 2,048 tokens with 32 heads of 128 takes 40 + 219 us with the rule of a decay per head (token by token
 // 1,242, 16 columns a block), eight prompts of 1,804 tokens 63 + 137 us with a decay per channel (816) and 24 + 32 + 143 us as
@@ -293,6 +295,32 @@ __global__ void __launch_bounds__(256) chunk_prepare_kernel(const ChunkArgs g) {
 }
 
 // ----------------------------------------------------------------------------- the chunks in order
+__device__ __forceinline__ bool finite(float v) { return fabsf(v) < INFINITY; }
+__device__ __forceinline__ bool all_finite(const f32x4_t& v) { return finite(v[0]) & finite(v[1]) & finite(v[2]) & finite(v[3]); }
+
+// acc + L x as four MFMAs give it (step i takes the rows 4 g + i in ascending order), for L zero above its diagonal, but row t
+// over the rows s <= t alone: the zeros above the diagonal times a later token's infinity would be NaN.  Operands and result
+// lie as the MFMAs have them: lane 16 g + r holds L[r][4 g ..+ 3], and of x, acc and the result rows 4 g ..+ 3 of column r.  What
+// is not finite in an earlier row (with `own` in row t itself too) makes the result NaN, as infinities of both signs do that
+// a walk adds up channel by channel.
+__device__ __forceinline__ f32x4_t causal_product(const f32x4_t& l, const f32x4_t& x, f32x4_t acc, bool own, int lane) {
+  const int n16 = lane % 16, g4 = lane / 16;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll 1
+    for (int g = 0; g < 4; ++g) {
+      const int s = 4 * g + i;
+      const float xs = __shfl(x[i], 16 * g + n16, kWave);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int t = 4 * g4 + j;
+        const float ls = __shfl(l[i], 16 * g + t, kWave);
+        if (s <= t) acc[j] = finite(xs) || (s == t && !own) ? fmaf(ls, xs, acc[j]) : NAN;
+      }
+    }
+  return acc;
+}
+
 template <int DK, int RULE>
 __global__ void __launch_bounds__(256, 2) chunk_walk_kernel(const ChunkArgs g, int column_groups) {
   constexpr bool kDelta = RULE == kRuleHead || RULE == kRuleChannel, kMemory = RULE == kRuleMemory;
@@ -373,12 +401,17 @@ __global__ void __launch_bounds__(256, 2) chunk_walk_kernel(const ChunkArgs g, i
 #pragma unroll
       for (int w = 1; w < 4; ++w) ks += parts[c & 1][w][1][lane];
       const f32x4_t r = u - ks;
+      const bool odd = __ballot(!all_finite(r)) != 0;  // (of all lanes: every wave has the same r)
       u = zero;
 #pragma unroll
       for (int i = 0; i < 4; ++i) u = mfma_f32(o.t[i], r[i], u);
-    }
 #pragma unroll
-    for (int x = 0; x < KT; ++x) S[x] *= o.last[x];
+      for (int x = 0; x < KT; ++x) S[x] *= o.last[x];  // (before the branch: while the MFMAs run)
+      if (odd) u = causal_product(o.t, r, zero, false, lane);
+    } else {
+#pragma unroll
+      for (int x = 0; x < KT; ++x) S[x] *= o.last[x];
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -387,8 +420,10 @@ __global__ void __launch_bounds__(256, 2) chunk_walk_kernel(const ChunkArgs g, i
       f32x4_t out = parts[c & 1][0][0][lane];
 #pragma unroll
       for (int w = 1; w < 4; ++w) out += parts[c & 1][w][0][lane];
+      const f32x4_t before = out;
 #pragma unroll
       for (int i = 0; i < 4; ++i) out = mfma_f32(o.p[i], u[i], out);
+      if (__ballot(!all_finite(out))) out = causal_product(o.p, u, before, kMemory, lane);  // (its walk reads the state that has the token; the others add q . k u)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int t = t0 + 4 * g4 + i;
