@@ -3,7 +3,7 @@ a sampled row, and which matrix-product kernel a tuned table sends a product to.
 
 import torch
 
-from torchllms_amd.kernels import attention_ops, ops, products
+from torchllms_amd.kernels import attention_ops, ops, products, sequence_ops
 
 
 def test_decode_splits_cover_the_range_and_stay_under_a_cu_s_share_of_blocks():
@@ -45,6 +45,28 @@ def test_requests_of_512_keys_and_fewer_are_left_whole_from_half_a_pair_a_cu_on(
         assert ops.decode_splits(16, 8, 512, head_dim) == ops.decode_splits(128, 1, 100, head_dim, uneven=True) == (512, 1)
     for args in ((16, 8, 513, 64), (15, 8, 512, 128), (16, 8, 512, 256)):  # longer, fewer, or wider heads: as planned
         assert ops.decode_splits(*args) == ops.plan_decode_splits(*args)
+
+
+def test_recurrences_are_walked_where_the_workspace_of_the_chunks_is_too_large_or_not_to_be_had(monkeypatch):
+    sizes = []
+
+    class Library:
+        @staticmethod
+        def tl_chunk_floats(n, rows, heads, dim, memory):
+            sizes.append((n, rows, heads, dim, memory))
+            return 1000 if rows < 50 else sequence_ops.CHUNK_FLOATS_MOST + 1
+
+    monkeypatch.setattr(sequence_ops, "core", lambda: Library)
+    args = dict(n_heads=2, head_dim=64, device="cpu")
+    ws, floats = sequence_ops._chunk_workspace(torch.bfloat16, 16, 3, 40, 5, **args)
+    assert ws.numel() == floats == 1000 and ws.dtype == torch.float32 and sizes == [(37, 2, 2, 64, 0)]
+    assert sequence_ops._chunk_workspace(torch.bfloat16, 16, 0, 2000, 50, **args) == (None, 0)
+
+    def full(*_, **__):
+        raise torch.OutOfMemoryError("full")
+
+    monkeypatch.setattr(torch, "empty", full)
+    assert sequence_ops._chunk_workspace(torch.bfloat16, 16, 3, 40, 5, **args) == (None, 0)
 
 
 def test_a_sampled_row_is_cut_only_when_rows_are_few_and_long():

@@ -24,7 +24,8 @@
 // 1,242, 16 columns a block), eight prompts of 1,804 tokens 63 + 137 us with a decay per channel (816) and 24 + 32 + 143 us as
 // matrix memory (634).  Against 64 bits (states after 40 to 2,089 tokens, all four kinds): 0.92 to 1.3 times the walk's distance,
 // on average just below it.
-// The workspace is bounded by walking a step's tokens in windows (the state goes through memory between them).
+// The workspace grows with the rows: a step's tokens are taken in windows (the state goes through memory between them), and it
+// holds a slot for every 16 tokens of a window and one more for every row of the step.  The caller bounds it, or walks.
 #include "common.h"
 #include "recurrence.h"
 

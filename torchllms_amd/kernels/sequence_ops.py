@@ -310,13 +310,20 @@ def selective_scan(
     return out
 
 
-#: the longest row of a step from which on prompts' rows of a bfloat16 step go by chunks of 16 tokens, and the most 32-bit
-#: numbers a step takes for that (a gigabyte: a step of so many rows is walked)
-CHUNKS_FROM, CHUNK_FLOATS_MOST = 16, 1 << 28
+#: the longest row of a step from which on prompts' rows of a bfloat16 step go by chunks of 16 tokens.  Chunks | walk, us, delta
+#: rule and matrix memory of 32 heads of 128: 8 rows of 2 tokens 40 | 39 and 41 | 35, of 8 41 | 47 and 42 | 47, of 16 42 | 58 and
+#: 42 | 62; 256 rows of 2 tokens 740 | 1,002 and 606 | 928, of 16 883 | 1,664 and 762 | 1,799.  A long row beside many short ones
+#: (16 tokens and 256 rows of 2: 743 | 1,006 and 612 | 936) takes them all along to their gain.
+CHUNKS_FROM = 16
+#: the most 32-bit numbers a layer's call takes for that from torch's allocator (a gigabyte; a step of more rows is walked:
+#: with 32 heads of 128 that is 1,236 slots, one a row and one for every 16 tokens of a window of 2,048)
+CHUNK_FLOATS_MOST = 1 << 28
 
 
 def _chunk_workspace(dtype: torch.dtype, longest: int, single_rows: int, n: int, n_seqs: int, n_heads: int, head_dim: int, device, memory: bool = False):
-    """``(workspace or None, its size)`` of a step whose longest row brings ``longest`` tokens."""
+    """``(workspace or None, its size)`` of a step whose longest row brings ``longest`` tokens.  Pools may have been given
+    nearly all of the memory: where it does not hold the workspace beside the results (allocate those first), the rows are
+    walked, which takes none."""
     if not 0 <= single_rows <= n_seqs:
         raise KernelError(f"{single_rows} rows of one token among {n_seqs} rows")
     if dtype != torch.bfloat16 or longest < CHUNKS_FROM or n <= n_seqs:
@@ -324,7 +331,10 @@ def _chunk_workspace(dtype: torch.dtype, longest: int, single_rows: int, n: int,
     floats = core().tl_chunk_floats(n - single_rows, n_seqs - single_rows, n_heads, head_dim, 1 if memory else 0)
     if not 0 < floats <= CHUNK_FLOATS_MOST:
         return None, 0
-    return torch.empty(floats, dtype=torch.float32, device=device), floats
+    try:
+        return torch.empty(floats, dtype=torch.float32, device=device), floats
+    except torch.OutOfMemoryError:
+        return None, 0
 
 
 def gated_delta(
@@ -390,9 +400,9 @@ def gated_delta(
             raise KernelError(f"gated_delta: a float32 vector of {size} entries expected, got {tuple(v.shape)} {v.dtype}")
     n_seqs = _step_rows(None, qo_indptr, slot_ids, n, state)
     region, stride = state_region(state, state_offset, H * dv * dk)
-    ws, floats = _chunk_workspace(qkv.dtype, longest, single_rows, n, n_seqs, H, dk, qkv.device)
     out = torch.empty((n, H * dv), dtype=qkv.dtype, device=qkv.device)
     o_raw = torch.empty((n, H * dv), dtype=torch.float32, device=qkv.device)
+    ws, floats = _chunk_workspace(qkv.dtype, longest, single_rows, n, n_seqs, H, dk, qkv.device)
     check(
         core().tl_gated_delta(
             qkv.data_ptr(), qkv.stride(0), proj.data_ptr(), proj.stride(0), gate_offset, b_offset, a_offset, A_log.data_ptr(),
@@ -447,9 +457,9 @@ def gated_linear(
         raise KernelError("gated_linear: the decay's power must be positive")
     n_seqs = _step_rows(None, qo_indptr, slot_ids, n, state)
     region, stride = state_region(state, state_offset, H * dv * dk)
-    ws, floats = _chunk_workspace(qkv.dtype, longest, single_rows, n, n_seqs, H, dk, qkv.device)
     out = torch.empty((n, H * dv), dtype=qkv.dtype, device=qkv.device)
     o_raw = torch.empty((n, H * dv), dtype=torch.float32, device=qkv.device)
+    ws, floats = _chunk_workspace(qkv.dtype, longest, single_rows, n, n_seqs, H, dk, qkv.device)
     check(
         core().tl_gated_delta(
             qkv.data_ptr(), qkv.stride(0), None, 0, gate_offset, 0, 0, None, decay_bias.data_ptr(), norm_weight.data_ptr(), float(eps),
@@ -515,10 +525,10 @@ def matrix_memory(
         raise KernelError("matrix_memory: the gates' cap must be positive")
     n_seqs = _step_rows(None, qo_indptr, slot_ids, n, state)
     region, stride = state_region(state, state_offset, matrix_memory_state_size(H, dk, dv))
-    ws, floats = _chunk_workspace(proj.dtype, longest, single_rows, n, n_seqs, H, dk, proj.device, memory=True)
     out = torch.empty((n, H * dv), dtype=proj.dtype, device=proj.device)
     o_raw = torch.empty((n, H * dv), dtype=torch.float32, device=proj.device)
     den = torch.empty((n, H), dtype=torch.float32, device=proj.device)
+    ws, floats = _chunk_workspace(proj.dtype, longest, single_rows, n, n_seqs, H, dk, proj.device, memory=True)
     check(
         core().tl_matrix_memory(
             proj.data_ptr(), proj.stride(0), q_offset, k_offset, v_offset, i_offset, f_offset, i_bias.data_ptr(), f_bias.data_ptr(),
