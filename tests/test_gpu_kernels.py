@@ -355,6 +355,17 @@ def test_gemm_f32_tiles_give_the_bits_of_the_kernel_for_few_rows(m, n, k, aligne
         assert torch.equal(_ops().gemm_f32(x[first : first + 9], w), got[first : first + 9])
 
 
+@pytest.mark.parametrize("m, n, k", [(17, 65536 * 32, 4), (17, 65536 * 32 + 5, 3)])
+def test_gemm_f32_of_more_columns_than_a_grid_has_rows_of_tiles(m, n, k):
+    """More than 65,535 tiles of 32 columns, aligned rows and others: chains of k fused multiply-adds."""
+    torch.manual_seed(n)
+    x, w = torch.randn(m, k, device=DEV), torch.randn(n, k, device=DEV)
+    got = _ops().gemm_f32(x, w)
+    for at in (slice(0, 64), slice(n // 2, n // 2 + 64), slice(n - 64, n)):
+        bound = k * 2.0 ** -24 * (x.double().abs() @ w[at].double().abs().T)
+        assert bool(((got[:, at].double() - x.double() @ w[at].double().T).abs() <= bound).all())
+
+
 # ----------------------------------------------------------------------------- layer norm
 @pytest.mark.parametrize("hidden", [4, 5, 1020, 1024, 1028, 2052, 4096, 8192, 8196])
 @pytest.mark.parametrize("stream, out", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16), (torch.bfloat16, torch.bfloat16)])

@@ -60,7 +60,8 @@ gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __restri
   const int wave = tid / kWave, lane = tid % kWave;
   const int n16 = lane % 16, g4 = lane / 16;
   // consecutive blocks share their columns: the tile of W is read from memory once for all of them
-  const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
+  const unsigned row_tiles = (unsigned)(M + BM - 1) / BM;
+  const int m0 = (int)(blockIdx.x % row_tiles) * BM, n0 = (int)(blockIdx.x / row_tiles) * BN;
   const int wm = (wave % (BM / WM)) * WM, wn = (wave / (BM / WM)) * WN;
   const int steps = (K + kStepF - 1) / kStepF;
 
@@ -381,14 +382,14 @@ gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __restri
 template <int BM, int WM, int kStepF, int kStages, bool kVec>
 int launch_tile(const float* A, int lda, const float* W, int ldw, float* C, int ldc, int M, int N, int K, hipStream_t stream) {
   constexpr size_t kLds = (size_t)kStages * (2 * BM) * kStepF * sizeof(float);
-  const dim3 grid((M + BM - 1) / BM, (N + BM - 1) / BM);
-  TL_REQUIRE(grid.y <= 65535, "gemm_f32: N=%d exceeds the grid limit of one launch", N);
+  const size_t grid = ((size_t)M + BM - 1) / BM * (((size_t)N + BM - 1) / BM);  // (one dimension: the others end at 65,535 tiles)
+  TL_REQUIRE(grid * 256 < (1ull << 32), "gemm_f32: %d x %d exceeds the grid limit of one launch", M, N);
   if (kLds > 48 * 1024) {
     hipError_t e = hipFuncSetAttribute((const void*)gemm_f32_tile_kernel<BM, BM, WM, WM, kStepF, kStages, kVec>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds);
     if (e != hipSuccess) return tl_fail(TL_ERR_HIP, "gemm_f32: %s", hipGetErrorString(e));
   }
-  gemm_f32_tile_kernel<BM, BM, WM, WM, kStepF, kStages, kVec><<<grid, 256, kLds, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+  gemm_f32_tile_kernel<BM, BM, WM, WM, kStepF, kStages, kVec><<<dim3((unsigned)grid), 256, kLds, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
   return tl_check_launch("gemm_f32_tile");
 }
 
