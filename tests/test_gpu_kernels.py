@@ -426,6 +426,31 @@ def test_expert_products_by_tiles(counts, D, F):
         assert bool(((y[at].double() - x @ w.T).abs() <= F * 2.0 ** -24 * (x.abs() @ w.abs().T) + 1e-30).all())
 
 
+def test_expert_products_of_tensors_off_a_16_byte_boundary():
+    """They take the kernels without LDS loads: the same products within the roundings of sums in another order, and an error
+    where dense layers' roundings are asked for."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(3)
+    offsets, D, F = _i32([0, 20, 20, 50]), 128, 64
+
+    def off(t):
+        flat = torch.empty(t.numel() + 4, dtype=t.dtype, device=DEV)
+        flat[4:] = t.reshape(-1).to(DEV)
+        return flat[4:].view(t.shape)
+
+    rows, gu, down = ((torch.randn(*s, generator=g) * k).bfloat16() for s, k in (((50, D), 1.0), ((3, 2 * F, D), 0.1), ((3, D, F), 0.1)))
+    mid = ops.expert_glu_rows(rows.to(DEV), gu.to(DEV), offsets)
+    y = ops.expert_down_rows(mid, down.to(DEV), offsets)
+    for x, w in ((off(rows), gu.to(DEV)), (rows.to(DEV), off(gu))):
+        got = ops.expert_glu_rows(x, w, offsets)
+        assert bool(((got.float() - mid.float()).abs() <= 2.0 ** -7 * mid.float().abs() + 1e-6).all())
+        with pytest.raises(ops.KernelError):
+            ops.expert_glu_rows(x, w, offsets, rounded=True)
+    slack = 2 * F * 2.0 ** -24 * F * mid.float().abs().max().item() * down.float().abs().max().item()  # F roundings a side of F products
+    for x, w in ((off(mid), down.to(DEV)), (mid, off(down))):
+        assert bool(((ops.expert_down_rows(x, w, offsets) - y).abs() <= slack).all())
+
+
 @pytest.mark.parametrize("tokens, E, D, F, prompt", [(256, 8, 256, 192, True), (600, 4, 320, 128, True), (1030, 3, 64, 5184, True),
                                                      (255, 8, 256, 192, True), (600, 4, 320, 128, False)])
 def test_routed_experts_of_prompts_round_as_dense_layers(tokens, E, D, F, prompt):

@@ -385,8 +385,11 @@ int launch_expert_wide(const void* rows, const void* w, const int32_t* offsets, 
 
 }  // namespace
 
-// Sizes the kernel takes: K a multiple of a step, columns in fours.
-bool tl_expert_tiles_fit(int K, int N) { return K % kStepE == 0 && N % 4 == 0; }
+// What the kernels take: K a multiple of a step, columns in fours, rows and weights on 16-byte boundaries (K in 64s keeps every row
+// there), results on those of their stores.
+bool tl_expert_tiles_fit(const void* rows, const void* w, const void* mid, const float* y, int K, int N) {
+  return K % kStepE == 0 && N % 4 == 0 && ((uintptr_t)rows | (uintptr_t)w | (uintptr_t)y) % 16 == 0 && (uintptr_t)mid % 8 == 0;
+}
 
 // mid != null: the gated product (w [E, 2 N, K], gate rows then up rows; rounded: as dense layers do), otherwise y = the plain one
 // (w [E, N, K]).

@@ -872,20 +872,20 @@ static int outputs_per_block(int n_experts, int n_out, int max_rows) {
   return per < waves ? waves : per;
 }
 
-// rows [pairs, D] in the order of their experts, offsets [n_experts + 1 ..]; mid [pairs, F].
-// (gemm_experts.hip)
-bool tl_expert_tiles_fit(int K, int N);
+// (gemm_experts.hip) Do the tiles take these sizes and addresses: what they fetch goes to LDS 16 bytes a lane.
+bool tl_expert_tiles_fit(const void* rows, const void* w, const void* mid, const float* y, int K, int N);
 int tl_expert_tiles(const void* rows, const void* w, const int32_t* offsets, int n_experts, void* mid, float* y, int K, int N, int pairs,
                     bool rounded, hipStream_t stream);
 
+// rows [pairs, D] in the order of their experts, offsets [n_experts + 1 ..]; mid [pairs, F].  rounded: see gemm_experts.hip.
 TL_EXPORT int tl_expert_glu_rows(const void* rows, const void* w_gu, const int32_t* offsets, int n_experts, void* mid, int D, int F,
                                  int max_rows, int dtype, int rounded, hipStream_t stream) {
   TL_REQUIRE(n_experts >= 0 && D > 0 && F > 0 && max_rows >= 0, "expert_glu_rows: bad sizes");
   if (n_experts == 0 || max_rows == 0) return TL_OK;
   if (dtype != TL_F32 && dtype != TL_BF16) return tl_fail(TL_ERR_ARG, "expert_glu_rows: unknown dtype %d", dtype);
-  if (dtype == TL_BF16 && tl_expert_tiles_fit(D, F))
+  if (dtype == TL_BF16 && tl_expert_tiles_fit(rows, w_gu, mid, nullptr, D, F))
     return tl_expert_tiles(rows, w_gu, offsets, n_experts, mid, nullptr, D, F, max_rows, rounded != 0, stream);
-  if (rounded) return tl_fail(TL_ERR_UNSUPPORTED, "expert_glu_rows: dense layers' roundings are for bfloat16 and widths that the tiles take");
+  if (rounded) return tl_fail(TL_ERR_UNSUPPORTED, "expert_glu_rows: dense layers' roundings are for bfloat16, widths in 64s and tensors on 16-byte boundaries");
   if (dtype == TL_BF16 && D % 8 == 0 && D <= kHeldMaxWidth)
     return launch_rows_held<true>(rows, w_gu, offsets, n_experts, mid, nullptr, D, F, max_rows, stream);
   const int elem = dtype == TL_F32 ? 4 : 2;
@@ -913,7 +913,7 @@ TL_EXPORT int tl_expert_down_rows(const void* mid, const void* w_d, const int32_
   TL_REQUIRE(n_experts >= 0 && D > 0 && F > 0 && max_rows >= 0, "expert_down_rows: bad sizes");
   if (n_experts == 0 || max_rows == 0) return TL_OK;
   if (dtype != TL_F32 && dtype != TL_BF16) return tl_fail(TL_ERR_ARG, "expert_down_rows: unknown dtype %d", dtype);
-  if (dtype == TL_BF16 && tl_expert_tiles_fit(F, D))
+  if (dtype == TL_BF16 && tl_expert_tiles_fit(mid, w_d, nullptr, y, F, D))
     return tl_expert_tiles(mid, w_d, offsets, n_experts, nullptr, y, F, D, max_rows, false, stream);
   if (dtype == TL_BF16 && F % 8 == 0 && F <= kHeldMaxWidth)
     return launch_rows_held<false>(mid, w_d, offsets, n_experts, nullptr, y, F, D, max_rows, stream);
