@@ -258,7 +258,7 @@ def plan_decode_splits(n_tokens: int, n_kv_heads: int, longest: int, head_dim: i
 
 #: up to this many keys a batch of two and more (request, kv head) pairs a CU is left whole, however uneven
 _DECODE_WHOLE_UNEVEN = 1024
-#: up to this many keys (the least a recorded step is made for) a batch of a pair for every second CU is left whole
+#: up to this many keys (the least a recorded step is made for) a batch of five pairs for eight CUs is left whole
 _DECODE_WHOLE_SHORT = 512
 
 
@@ -269,12 +269,13 @@ def decode_splits(n_tokens: int, n_kv_heads: int, longest: int, head_dim: int = 
     and merge, split at 512 keys | left whole: head size 128 up to 750 keys 39.8 | 29.1 us, up to 1,000 43.5 | 36.8, up to
     1,500 55.1 | 53.6, up to 2,000 68.9 | 69.3; head size 64 27.5 | 20.7, 28.1 | 26.0, 35.2 | 37.0, 40.0 | 47.4.)
 
-    Up to 512 keys half as many pairs are enough: a recorded step is made for 512 keys also where its requests hold a
-    hundred, and then most splits are empty and the merge is for nothing.  (As planned | whole, us, a step for 512 keys, requests
-    of 100, 256 and 512: head size 128, 16 requests of 8 kv heads 11.5 | 7.3, 13.8 | 10.5, 15.9 | 16.4, 24 requests 11.8 | 7.7,
-    17.2 | 11.7, 19.0 | 18.5; head size 64 9.4 | 5.8, 9.8 | 8.4, 11.1 | 13.3 and 10.8 | 6.0, 12.5 | 8.8, 13.4 | 13.7; of fewer
-    requests the longest lose more than the shortest gain: 8 of head size 64 8.2 | 5.6, 8.4 | 7.4, 8.6 | 11.6.)"""
-    if longest <= _DECODE_WHOLE_SHORT and head_dim <= 128 and 2 * n_tokens * n_kv_heads >= device_facts()[0]:
+    Up to 512 keys five pairs for eight CUs are enough: a recorded step is made for 512 keys also where its requests hold a
+    hundred, and then most splits are empty and the merge is for nothing.  The line lies where requests that do hold 512 keys
+    lose nothing.  (As planned | whole, us, a step for 512 keys, 8 kv heads, requests of 100, 256, 384 and 512: head size 128, 20
+    requests 11.5 | 7.2, 13.9 | 9.8, 14.5 | 12.8, 17.0 | 16.3, 24 requests 11.5 | 7.4, 15.3 | 10.2, 17.6 | 13.9, 18.5 | 18.4; head
+    size 64, 20 requests 10.7 | 5.9, 11.3 | 7.9, 11.5 | 9.7, 12.1 | 11.6, 32 requests 11.0 | 6.0, 13.1 | 8.1, 13.5 | 10.2, 14.7 |
+    13.4; but 16 requests 9.3 | 5.7, 9.8 | 7.8, 10.0 | 9.6, 10.4 | 11.5, and of head size 32 the last 9.6 | 10.4.)"""
+    if longest <= _DECODE_WHOLE_SHORT and head_dim <= 128 and 8 * n_tokens * n_kv_heads >= 5 * device_facts()[0]:
         return _DECODE_WHOLE_SHORT, 1
     many = n_tokens * n_kv_heads >= 2 * device_facts()[0]
     return plan_decode_splits(n_tokens, n_kv_heads, longest, head_dim, uneven=uneven and not (many and longest <= _DECODE_WHOLE_UNEVEN))
