@@ -48,6 +48,16 @@ def test_requests_of_512_keys_and_fewer_are_left_whole_from_five_pairs_for_eight
         assert ops.decode_splits(*args) == ops.plan_decode_splits(*args)
 
 
+def test_32_bit_prompts_take_the_matrix_cores_where_few_requests_meet_in_a_block():
+    one, eights, ragged = [0, 562], [8 * i for i in range(33)], [3, 25, 30, 400, 700]
+    for heads, kv, dim, bounds, longest, want in (
+            (32, 8, 64, one, 562, True), (32, 8, 128, one, 562, True), (6, 2, 128, one, 562, True), (4, 4, 32, [0, 33], 33, True),
+            (8, 8, 128, eights, 8, False), (6, 2, 64, eights, 508, False), (8, 1, 128, eights, 508, False),  # 8, 8 and 2 meet
+            (64, 8, 64, eights, 508, True), (32, 8, 64, [0, 32], 32, False), (32, 8, 128, [0, 64], 64, False),  # blocks for every CU; few keys
+            (32, 8, 64, ragged, 700, True), (8, 8, 64, ragged, 700, False)):
+        assert ops.runs_on_end(bounds, heads, kv, dim, longest) is want, (heads, kv, dim, bounds[-1], longest)
+
+
 def test_recurrences_are_walked_where_the_workspace_of_the_chunks_is_too_large_or_not_to_be_had(monkeypatch):
     sizes = []
 

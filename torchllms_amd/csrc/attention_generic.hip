@@ -795,8 +795,8 @@ attention_join_kernel(T* __restrict__ out, int out_stride, const int32_t* __rest
 // pages: [page][n_kv_heads][page_size][head_dim].  token_seq[t]: row of block_table;
 // positions[t]: absolute position; the token sees positions max(0, p-window+1)..p (window 0: all).  slopes: one float
 // per query head (or null) that a capped score loses for every position between its key and the query; dist: a table
-// [n_q_heads][dist_len] (or null) of what it gains by distance instead.  on_end: tokens stand in runs of many of one request
-// (prompts); the result is the same either way.
+// [n_q_heads][dist_len] (or null) of what it gains by distance instead.  on_end: take the matrix cores where their kernel
+// is built for the sizes (tokens in long runs of one request); the result is the same either way.
 TL_EXPORT int tl_attention_generic(const void* q, int q_stride, void* out, int out_stride,
                                    const void* k_pages, const void* v_pages, const int32_t* token_seq,
                                    const int32_t* positions, const int32_t* block_table, int bt_stride,
@@ -825,9 +825,9 @@ TL_EXPORT int tl_attention_generic(const void* q, int q_stride, void* out, int o
   const bool vec = head_dim % 4 == 0 && v_dim % 4 == 0 && v_pitch % 4 == 0 && ((uintptr_t)k_pages % 16) == 0 && ((uintptr_t)v_pages % 16) == 0;
   // prompt portions: tokens and heads that read the same keys share them through LDS (same bits)
   const size_t tile_lds = ((size_t)kTileWaves * head_dim + (size_t)kWave * (head_dim + v_dim + 2 * kTilePad)) * sizeof(float);
-  // ... in 32-bit on the matrix cores (a third of the time of the shared tiles, see there), if many tokens on end belong to a
-  // request (a block works off one request after the other, so that runs of one or two would wait for each other; whoever
-  // calls knows) and the sizes are those the kernel is built for
+  // ... in 32-bit on the matrix cores (a third of the time of the shared tiles for a prompt, see there), if whoever calls says so
+  // (a block works off one request after the other, so that short runs wait for each other: runs_on_end in
+  // kernels/attention_ops.py) and the sizes are those the kernel is built for
   if (dtype == TL_F32 && on_end && n_tokens >= kTileMinTokens && vec && v_dim == head_dim && v_pitch == v_dim && n_v_heads == n_kv_heads &&
       (keep_first == 0 || (window == 0 && chunk == 0)) && (head_dim == 16 || head_dim == 32 || head_dim == 64 || head_dim == 128)) {
     const int group = n_q_heads / n_kv_heads;

@@ -13,11 +13,6 @@ from . import ops
 
 #: contexts beyond this many keys give every block of 64 keys a wave of its own in the plain kernel
 GENERIC_SPLIT_FROM = 128
-#: prompt portions of this many tokens each on average count as runs on end for the plain kernel: a block of its 32-bit form
-#: for the matrix cores takes 16 tokens or more, one request after the other.  256 tokens of 32 heads of 64 behind 64 | 512 |
-#: 2,048 keys, us, shared tiles and matrix cores: portions of 4 tokens 30 and 43 | 140 and 170 | 570 and 609, of 8 tokens 32 and
-#: 25 | 142 and 89 | 531 and 306, of 16 31 and 18 | 142 and 48 | 516 and 156; heads of 128 cross at the same place.
-GENERIC_ON_END = 8
 
 
 def paged_attention(
@@ -135,9 +130,16 @@ def paged_attention(
                     **(dict(v_offset=at) if at or v_dim != head_dim else {}),
                 )
         else:
+            on_end = False
+            if qkv.dtype == torch.float32:
+                key = ("on_end", n_q_heads, n_kv_heads, head_dim, window, chunk)
+                on_end = ctx.scratch.get(key)
+                if on_end is None:
+                    host = ctx.host
+                    longest = min(int(max(host.kv_lens[n_dec : host.n_seqs])), window or 1 << 30, chunk or 1 << 30)
+                    on_end = ctx.scratch[key] = ops.runs_on_end(host.qo_indptr[n_dec : host.n_seqs + 1], n_q_heads, n_kv_heads, head_dim, longest)
             ops.attention_generic(
                 qkv[n_dec:], n_q_heads, n_kv_heads, head_dim, k_pages, v_pages, ctx.token_seq[n_dec:],
-                ctx.positions[n_dec:], ctx.block_tables[group], window, scale, out=out[n_dec:],
-                on_end=n - n_dec >= GENERIC_ON_END * (ctx.host.n_seqs - n_dec), **extras,
+                ctx.positions[n_dec:], ctx.block_tables[group], window, scale, out=out[n_dec:], on_end=on_end, **extras,
             )
     return out

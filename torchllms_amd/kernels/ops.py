@@ -94,6 +94,7 @@ from .attention_ops import (  # noqa: F401
     plan_decode_splits,
     prefill_attention_supported,
     prefill_key_groups,
+    runs_on_end,
     prefill_queries_per_tile,
     prefill_tile_count,
     prefill_tiles,
