@@ -703,7 +703,7 @@ def attention_run(args, shape) -> int:
                     ops.attention_decode(q, hq, hkv, dh, k, v, seq, pos, tables, 0, dh ** -0.5, ctx, split_size=split)
 
                 row["planned" if split is None else str(split)] = round(_cold_graph_us(step, layers, flush) - base, 1)
-            plan = ops.plan_decode_splits(batch, hkv, ctx, dh)
+            plan = ops.decode_splits(batch, hkv, ctx, dh)
             mb = batch * ctx * hkv * dh * 4 / 1e6
             table[f"b{batch}_ctx{ctx}"] = {"plan": list(plan), "mb": round(mb, 1), "us": row}
             del caches

@@ -1,5 +1,6 @@
 """Recurrences over matrix states by chunks of 16 tokens (``csrc/delta_chunks.hip``) against the recurrences themselves in
-64 bits, and beside the token-by-token kernels: the chunks may be no further off than those are."""
+64 bits, and beside the token-by-token kernels: the chunks are about as far off as those (0.85 to 1.3 times over a step's
+states, 0.97 on average), which the bounds hold them to row by row and head by head."""
 
 from __future__ import annotations
 
@@ -36,17 +37,20 @@ def _over_rms(o):
     return o / torch.sqrt((o * o).mean(-1, keepdim=True) + EPS)
 
 
-def _check(outs, states, want, want_states, offsets):
-    """``outs`` = (by chunks, walked): results within the rounding to bfloat16 and 32-bit sums of the 64-bit ones, and the
-    states of the chunks as near as the walk's (twice its distance: sums in another order) or within 2e-6 of them."""
+def _check(outs, states, want, want_states, offsets, heads, chunked=True):
+    """``outs`` = (by chunks, walked): results within the rounding to bfloat16 and 32-bit sums of the 64-bit ones, and every
+    row's state of every head as near as the walk's: one and a half times its distance (sums in another order) and two
+    roundings.  ``heads``: a state row is [heads, ..]."""
     assert not bool(torch.isnan(outs[0].float()).any())
     for r in range(offsets.numel() - 1):
         at = slice(int(offsets[r]), int(offsets[r + 1]))
         scale = want[at].abs().max()
         assert (outs[0][at].double() - want[at]).abs().max() <= 2.0 ** -8 * scale + 2 * (outs[1][at].double() - want[at]).abs().max()
-    norm = want_states.norm()
-    err = [(s.double() - want_states).norm() / norm for s in states]
-    assert err[0] <= 2 * err[1] + 2e-6, err
+    truth = want_states.view(want_states.shape[0], heads, -1)
+    err = [(s.double().view(truth.shape) - truth).norm(dim=-1) / truth.norm(dim=-1) for s in states]
+    assert bool((err[0] <= 1.5 * err[1] + 2.0 ** -23).all()), err
+    if chunked:  # (and they did go by chunks: sums in another order)
+        assert not torch.equal(states[0], states[1])
 
 
 LENGTHS = [[1, 1, 16, 1, 17, 33], [15, 1, 130, 31], [250], [2049 + 40]]
@@ -54,10 +58,11 @@ LENGTHS = [[1, 1, 16, 1, 17, 33], [15, 1, 130, 31], [250], [2049 + 40]]
 
 @pytest.mark.parametrize("rule", ["head", "channel", "plain"])
 @pytest.mark.parametrize("lengths", LENGTHS)
-@pytest.mark.parametrize("H,G,dk,dv", [(2, 1, 64, 24), (8, 8, 128, 16), (3, 3, 64, 130)])
+@pytest.mark.parametrize("H,G,dk,dv", [(2, 1, 64, 24), (8, 8, 128, 16), (4, 4, 64, 130), (3, 3, 64, 130)])
 def test_delta_rule_and_linear_attention_by_chunks(rule, lengths, H, G, dk, dv):
     """Rows that end inside a chunk, rows of single tokens before them, a row beyond a window of tokens; decays near one,
-    decays that forget at once (and to zero exactly) beside them, in one channel or in all; a written key read back late."""
+    decays that forget at once (and to zero exactly) beside them, in one channel or in all; a written key read back late.  Rows
+    of an odd number of pairs (the last sizes) are walked."""
     from torchllms_amd.kernels import ops
 
     if rule == "plain":
@@ -115,14 +120,15 @@ def test_delta_rule_and_linear_attention_by_chunks(rule, lengths, H, G, dk, dv):
         want[at], last = _walk64(q[at], k[at], v[at], decay[at], None if beta is None else beta[at], s0)
         want_states[slots[r]] = last.transpose(1, 2).reshape(-1)
     want = (_over_rms(want) * norm_w.double()).reshape(n, -1) * torch.nn.functional.silu(gate.double())
-    _check(outs, states, want, want_states, offsets)
+    _check(outs, states, want, want_states, offsets, H, chunked=qkv.shape[1] % 4 == 0)
 
 
 @pytest.mark.parametrize("lengths", LENGTHS)
-@pytest.mark.parametrize("H,dk,dv", [(2, 64, 24), (8, 128, 16), (3, 64, 128)])
+@pytest.mark.parametrize("H,dk,dv", [(2, 64, 24), (8, 128, 16), (4, 64, 128), (3, 64, 128)])
 def test_matrix_memory_by_chunks(lengths, H, dk, dv):
     """Input gates that jump above the running maximum inside a chunk and far below it, forget gates that drop everything,
-    gates beyond the cap; the normaliser's column behind a full group of columns and inside one."""
+    gates beyond the cap; the normaliser's column behind a full group of columns and inside one.  Rows of an odd number of
+    pairs (the last sizes) are walked."""
     from torchllms_amd.kernels import ops
 
     lengths, offsets, singles = _rows(lengths)
@@ -170,7 +176,7 @@ def test_matrix_memory_by_chunks(lengths, H, dk, dv):
         matrices[slots[r]] = last.transpose(1, 2).reshape(-1)
         tops[slots[r]] = m
     want = _over_rms(want).reshape(n, -1) * norm_w.double() * torch.sigmoid(x[:, 2 * qk + vw : 2 * qk + 2 * vw])
-    _check(outs, [s[:, : H * (dv + 1) * dk] for s in states], want, matrices, offsets)
+    _check(outs, [s[:, : H * (dv + 1) * dk] for s in states], want, matrices, offsets, H, chunked=proj.shape[1] % 4 == 0)
     for s in states:
         top = s[:, H * (dv + 1) * dk : H * (dv + 1) * (dk + 1)].view(len(lengths), H, dv + 1).double()
         assert bool(((top - tops[..., None]).abs() <= 1e-5 * (1 + tops[..., None].abs())).all())

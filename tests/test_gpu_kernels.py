@@ -355,6 +355,32 @@ def test_gemm_f32_tiles_give_the_bits_of_the_kernel_for_few_rows(m, n, k, aligne
         assert torch.equal(_ops().gemm_f32(x[first : first + 9], w), got[first : first + 9])
 
 
+def _wide_range(*shape):
+    """Numbers whose exponents differ widely, denormal ones and zeros among them, so that products and sums are denormal,
+    vanish beside each other or cancel: rows of ordinary, large and tiny numbers, and of terms that take each other away."""
+    x = torch.randn(*shape, device=DEV)
+    x = torch.ldexp(x, torch.randint(-30, 31, shape, device=DEV))
+    x[1::7] = torch.ldexp(x[1::7], torch.tensor(-70, device=DEV))  # products of two such rows are denormal or nothing
+    x[2::7] = torch.ldexp(x[2::7], torch.tensor(-115, device=DEV))  # many are denormal already
+    x[3::7, 1::2] = -x[3::7, : shape[1] // 2 * 2 : 2]  # with equal numbers on the other side: sums that cancel
+    x[4::7] = torch.randn_like(x[4::7])
+    x[5::7, ::3] = 0.0
+    return x
+
+
+@pytest.mark.parametrize("m, n, k", [(40, 90, 64), (300, 700, 256), (1030, 4200, 64), (70, 64, 33)])
+def test_gemm_f32_tiles_keep_the_bits_of_denormal_and_cancelling_sums(m, n, k):
+    """The matrix cores round every step of a chain as fused multiply-adds do, whatever the exponents."""
+    torch.manual_seed(m + k)
+    x, w = _wide_range(m, k), _wide_range(n, k)
+    w[:, 1 : k // 2 * 2 : 2] = torch.where(torch.rand(n, 1, device=DEV) < 0.5, w[:, : k // 2 * 2 : 2], w[:, 1 : k // 2 * 2 : 2])
+    got = _ops().gemm_f32(x, w)
+    tiny = (got != 0) & (got.abs() < 2.0 ** -126)
+    assert bool(tiny.any()) and bool((got == 0).any()) and bool(torch.isfinite(got).all())
+    for first in range(0, m - 9, 9):
+        assert torch.equal(_ops().gemm_f32(x[first : first + 9], w).view(torch.int32), got[first : first + 9].view(torch.int32))
+
+
 @pytest.mark.parametrize("m, n, k", [(17, 65536 * 32, 4), (17, 65536 * 32 + 5, 3)])
 def test_gemm_f32_of_more_columns_than_a_grid_has_rows_of_tiles(m, n, k):
     """More than 65,535 tiles of 32 columns, aligned rows and others: chains of k fused multiply-adds."""
@@ -400,19 +426,30 @@ def test_layernorm_of_every_width(hidden, stream, out):
 @pytest.mark.parametrize("counts, D, F", [
     ([1], 64, 64), ([0, 3, 0, 17, 1, 0], 128, 192), ([15, 16, 17, 33], 64, 320), ([31, 0, 32, 65], 192, 64), ([64, 63, 129, 0, 65], 128, 448),
     ([127, 128, 129], 64, 192), ([300, 1, 0, 520], 320, 128), ([513], 64, 64), ([2, 0, 1] * 30, 64, 128), ([0, 0, 40] * 44, 64, 64),
-    ([600, 1, 255], 64, 5184), ([600, 1, 255], 10304, 64)])
+    ([600, 1, 255], 64, 5184), ([600, 1, 255], 192, 5184), ([600, 1, 255], 320, 5184), ([600, 1, 255], 3136, 5184), ([600, 1, 255], 10304, 64),
+    ([600, 1, 255], 10304, 192), ([600, 1, 255], 10304, 320), ([600, 1, 255], 10304, 3136)])
 def test_expert_products_by_tiles(counts, D, F):
     """Every tile size (chosen by the mean rows of an expert), experts without rows, one row, a tile's edge, columns that
-    are no multiple of a tile (with the large tiles of either product among them), one step along K, more experts than a wave has lanes, and rows behind the last expert's
-    (pairs of outputs that are no experts), which stay unwritten."""
+    are no multiple of a tile, one step along K, more experts than a wave has lanes, and rows behind the last expert's
+    (pairs of outputs that are no experts), which stay unwritten.  The last eight: the large tiles of the gated and of the plain
+    product, 2, 6, 10 and 98 steps along K (three buffers are filled in turn)."""
+    from torchllms_amd.kernels.base import BF16, _stream, check, core
+
     ops = _ops()
     g = torch.Generator().manual_seed(sum(counts) + D)
     E, rest = len(counts), 5
     rows = torch.randn(sum(counts) + rest, D, generator=g).bfloat16()
     gu, down = ((torch.randn(E, *s, generator=g) * 0.1).bfloat16() for s in ((2 * F, D), (D, F)))
     offsets = torch.tensor([0] + list(np.cumsum(counts)) + [sum(counts) + rest], dtype=torch.int32)
-    mid = ops.expert_glu_rows(rows.to(DEV), gu.to(DEV), offsets.to(DEV)).cpu()
-    y = ops.expert_down_rows(mid.to(DEV), down.to(DEV), offsets.to(DEV)).cpu()
+    rows, gu, down, at_device = rows.to(DEV), gu.to(DEV), down.to(DEV), offsets.to(DEV)
+    mid, y = ops.expert_glu_rows(rows, gu, at_device), ops.expert_down_rows(rows.new_zeros(rows.shape[0], F), down, at_device)
+    assert mid.shape == (rows.shape[0], F) and y.shape == rows.shape and y.dtype == torch.float32
+    mid.fill_(7.0)
+    y.fill_(7.0)
+    check(core().tl_expert_glu_rows(rows.data_ptr(), gu.data_ptr(), at_device.data_ptr(), E, mid.data_ptr(), D, F, rows.shape[0], BF16, 0, _stream()))
+    check(core().tl_expert_down_rows(mid.data_ptr(), down.data_ptr(), at_device.data_ptr(), E, y.data_ptr(), D, F, rows.shape[0], BF16, _stream()))
+    assert bool((mid[-rest:] == 7.0).all()) and bool((y[-rest:] == 7.0).all())
+    assert torch.equal(ops.expert_glu_rows(rows, gu, at_device)[:-rest], mid[:-rest])
     for e in range(E):
         at = slice(int(offsets[e]), int(offsets[e + 1]))
         x, w = rows[at].double(), gu[e].double()
@@ -681,18 +718,20 @@ def test_attention_window_edge(dtype, window):
     assert (got[-1].view(hq, dh) - v[inside, 0]).abs().max() < (1e-3 if dtype == torch.float32 else 3e-2)
 
 
-@pytest.mark.parametrize("odd_value", [False, True])
+@pytest.mark.parametrize("values", ["ordinary", "odd", "wide"])
 @pytest.mark.parametrize(
     "hq, hkv, dh, page, sizes, kw",
     [(8, 2, 64, 16, [(200, 130), (70, 70), (300, 5), (65, 2)], {}), (4, 4, 128, 5, [(150, 33)], dict(window=40)),
      (16, 2, 32, 8, [(64, 64), (129, 65)], dict(chunk=48, softcap=3.0)), (6, 3, 16, 3, [(100, 37), (20, 20)], dict(slopes=True)),
      (3, 1, 128, 16, [(90, 41)], dict(window=64, sinks=True)), (4, 1, 64, 16, [(140, 63)], dict(distances=True))],
 )
-def test_attention_generic_on_the_matrix_cores_gives_the_same_bits(hq, hkv, dh, page, sizes, kw, odd_value):
+def test_attention_generic_on_the_matrix_cores_gives_the_same_bits(hq, hkv, dh, page, sizes, kw, values):
     """Prompts of 32-bit models (on_end) take blocks of 64 keys through matrix instructions, in the order of the sums of the
     kernels that multiply one by one: every form that is accepted, groups of 1, 2, 3, 4 and 8 query heads, tokens that fill no
-    block, several requests in one.  A value that is not a number reaches the queries that see its key and no others."""
+    block, several requests in one.  A value that is not a number reaches the queries that see its key and no others; numbers
+    whose exponents lie far apart round alike."""
     torch.manual_seed(dh + page)
+    odd_value, wide_range = values == "odd", values == "wide"
     kw = dict(kw)
     window = kw.pop("window", 0)
     for name, shape in (("slopes", (hq,)), ("sinks", (hq,)), ("distances", (hq, 50))):
@@ -709,6 +748,9 @@ def test_attention_generic_on_the_matrix_cores_gives_the_same_bits(hq, hkv, dh, 
     seqs = [r for r, (S, sq) in enumerate(sizes) for _ in range(sq)]
     poss = [p for S, sq in sizes for p in range(S - sq, S)]
     q = torch.randn(len(seqs), hq * dh + 12, device=DEV)
+    if wide_range:  # scores that nearly tie, far apart and denormal; values that vanish beside each other
+        q, k_pages, v_pages = (torch.ldexp(t, torch.randint(-r, r // 3, t.shape, device=DEV)) for t, r in ((q, 12), (k_pages, 12), (v_pages, 100)))
+        v_pages[::2] = torch.ldexp(v_pages[::2], torch.tensor(-60, device=DEV))
     args = (q, hq, hkv, dh, k_pages, v_pages, _i32(seqs), _i32(poss), _i32(tables.tolist()), window, dh ** -0.5)
     want, got = (_ops().attention_generic(*args, on_end=on_end, **kw) for on_end in (False, True))
     assert torch.equal(torch.isnan(want), torch.isnan(got))
