@@ -19,11 +19,11 @@
 //     operands are asked for two chunks ahead.  A chunk with values that are not finite takes its two triangular products row
 //     by row (causal_product): a token's infinity reaches itself and later ones alone, as in the walk.  (The look at every
 //     chunk's values costs the delta rules 1 to 2%: 2,048 tokens 240 -> 242 us in all, 4 x 3,000 1,532 -> 1,561.)
-// What bounds it: the walk, a chain of one chunk behind the other (about 0.6 us each: 16 + 4 + 8 MFMAs of 32 cycles and a
-// barrier): a prompt of 2,048 tokens with 32 heads of 128 takes 40 + 219 us with the rule of a decay per head (token by token
-// 1,242, 16 columns a block), eight prompts of 1,804 tokens 63 + 137 us with a decay per channel (816) and 24 + 32 + 143 us as
-// matrix memory (634).  Against 64 bits (states after 40 to 2,089 tokens, all four kinds): 0.92 to 1.3 times the walk's distance,
-// on average just below it.
+// What bounds it: the walk, a chain of one chunk behind the other, about 1.7 us each, of which 16 + 4 + 8 MFMAs of 32 cycles are
+// 0.4; the rest is the way through LDS, the barrier and the operands' loads.  A prompt of 2,048 tokens with 32 heads of 128 takes
+// 40 + 219 us with the rule of a decay per head (token by token 1,242, 16 columns a block), eight prompts of 1,804 tokens 63 + 137 us
+// with a decay per channel (816) and 24 + 32 + 143 us as matrix memory (634).  Against 64 bits (states after 15 to 2,089 tokens, all
+// four kinds): 0.85 to 1.27 times the walk's distance over a step's states, 0.97 on average.
 // The workspace grows with the rows: a step's tokens are taken in windows (the state goes through memory between them), and it
 // holds a slot for every 16 tokens of a window and one more for every row of the step.  The caller bounds it, or walks.
 #include "common.h"

@@ -17,9 +17,10 @@
 //     (bound by reading W: many blocks with several steps in flight).
 //   * Blocks go to the eight XCDs in turn.  All row tiles of one (expert, column tile) go to the same XCD one after the
 //     other, so W is read from memory once and met again in that XCD's L2; an expert's column tiles are spread over all XCDs.
-// 8 experts of 4,096 x 3,584, gated + plain product: 16 pairs 119 us (a wave per 16 columns with operands straight from memory,
-// before: 156; the bytes of W at 6.1 TB/s: 101), 128 pairs 123 (235; 116), 4,096 pairs 518 (a library product per expert, with
-// the activation in a kernel of its own: 632, and the host waited for the offsets once a layer), 408 by the large tiles.
+// 8 experts, pairs spread by chance, gated + plain product, us (the kernels for other widths, or a library product per expert, the
+// activation in a kernel of its own and a wait of the host, which these took the place of): 4,096 x 3,584, 16 pairs 79 + 40 (116 +
+// 46; the bytes of W at 6.1 TB/s: 77 + 38), 128 pairs 83 + 44 (159 + 94), 4,096 pairs 294 + 181 (650 in all); 2,048 x 2,048, 16
+// pairs 28 + 16 (38 + 22), 128 pairs 28 + 17 (45 + 25), 4,096 pairs 106 + 81 (441).
 #include <type_traits>
 
 #include "common.h"
@@ -184,9 +185,9 @@ expert_tile_kernel(const bf16_t* __restrict__ rows, const bf16_t* __restrict__ w
   const int steps = K / kStepE;
   // rows of W lie a power of two apart, so blocks that walk K in step would all press on the same memory channels at once:
   // the column tiles start their walks at different steps and wrap around (the row tiles of one at the same step: they share
-  // W in L2, and a row's sums do not depend on where it lies).  Eight experts of 2,048 x 2,048, 48 pairs: gated + plain product
-  // 35 + 18.8 us in step, 27.3 + 16.0 like this; of 4,096 x 3,584 90 + 42 and 80.5 + 42; 256 pairs 36.6 + 21.5 and 28.9 + 20.2 (94 + 54 and 88 + 55).
-  // With 128 rows a tile blocks lose what they share of the rows (4,096 pairs 299 + 150, and 328 + 159)
+  // W in L2, and a row's sums do not depend on where it lies).  Eight experts of 2,048 x 2,048, gated + plain product, in step | like
+  // this: 48 pairs 35.3 + 19.2 us | 27.5 + 16.5, 256 pairs 37.1 + 22.7 | 29.3 + 22.0; of 4,096 x 3,584 92.0 + 42.8 | 81.6 + 42.6 and
+  // 94.1 + 48.8 | 89.3 + 50.6.  With 128 rows a tile blocks lose what they share of the rows (4,096 pairs 315 + 202 | 345 + 212).
   const int rot = BM <= 64 ? (n_tile * 5 + e * 3) % steps : 0;
   auto step_of = [&](int i) { return i + rot < steps ? i + rot : i + rot - steps; };
 #pragma unroll
@@ -394,13 +395,16 @@ bool tl_expert_tiles_fit(const void* rows, const void* w, const void* mid, const
 // mid != null: the gated product (w [E, 2 N, K], gate rows then up rows; rounded: as dense layers do), otherwise y = the plain one
 // (w [E, N, K]).
 //
-// Which tile: by the rows an expert has on average (`pairs` counts those of outputs that are no experts too).  Measured at
-// 8 experts, gated + plain product in us, widths 4,096 x 3,584 | 2,048 x 2,048, with 16, 32, 64 and 128 rows a tile:
-// 16 pairs 119 120 119 - | 48 48 54 -; 256 pairs (32 rows) 163 137 135 173 | 61 59 55 79; 1,024 pairs (128 rows) - - 227 235
-// | - - 84 87; 2,424 pairs (303 rows) - - 371 364 | - - 127 125; 4,096 pairs - - 592 518 | - - 195 195.  128 x 256 tiles where
-// they are more than five for four CUs, 128 x 128 and 128 x 256: 2,424 pairs 234 + 137 and 223 + 132, 4,096 pairs 308 + 147 and
-// 265 + 143; where they are fewer the CUs that get none weigh more (2,048 x 2,048, 288 of them for the plain product: 47 and 50;
-// 4,096 x 1,024 gated, 288: 82 and 87).  (128 x 256 tiles with K in steps of 64 and one block a CU: 585 at 4,096 pairs.)
+// Which tile: by the rows an expert has on average (`pairs` counts those of outputs that are no experts too).  Measured at 8
+// experts, pairs spread by chance, gated + plain product in us, tiles of 16 | 32 | 64 | 128 rows | 128 x 256:
+//   4,096 x 3,584: 16 pairs 81 + 42 | 80 + 42 | 82 + 42; 128 pairs 91 + 48 | 83 + 43 | 83 + 43 | 103 + 67; 256 pairs 113 + 64 | 94 + 54 |
+//   90 + 46 | 104 + 66; 1,024 pairs 171 + 107 (32) | 146 + 86 | 160 + 75 | 152 + 81; 2,424 pairs 238 + 137 (64) | 230 + 135 | 228 + 127;
+//   4,096 pairs 374 + 215 (64) | 313 + 200 | 287 + 180.
+//   2,048 x 2,048: 16 pairs 28 + 16 | 27 + 16 | 28 + 24; 256 pairs 39 + 25 | 35 + 22 | 29 + 25 | 46 + 37; 1,024 pairs 59 + 37 (32) | 50 + 35
+//   | 50 + 41 | 51 + 44; 2,424 pairs 77 + 49 (64) | 81 + 46 | 75 + 45; 4,096 pairs 120 + 72 (64) | 118 + 81 | 106 + 66.
+// 128 x 256 tiles where they are more than five for four CUs; with fewer the CUs that get none weigh more (4,096 x 1,024, 512 to
+// 2,424 pairs, gated: 72 to 77 with 128 rows, 79 to 83 with these), though not everywhere: 288 of them for the plain product
+// of 4,096 pairs of 2,048 x 2,048 take 66, and 128 x 128, which the rule takes, 81.
 int tl_expert_tiles(const void* rows, const void* w, const int32_t* offsets, int n_experts, void* mid, float* y, int K, int N, int pairs,
                     bool rounded, hipStream_t stream) {
   const double mean = (double)pairs / n_experts;

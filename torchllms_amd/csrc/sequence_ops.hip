@@ -1310,11 +1310,6 @@ TL_EXPORT int tl_selective_scan(const void* x, const void* dt_pre, int dt_dtype,
   return tl_fail(TL_ERR_ARG, "selective_scan: dtype %d with step sizes of dtype %d", dtype, dt_dtype);
 }
 
-// qkv, proj, out as the kernels describe; state: S^T of head h at state + slot * state_stride + h * dv * dk;
-// o_raw: workspace of n_tokens * H * dv floats.  gate: the matrix whose H * dv columns from gate_off hold the output
-// gate (proj itself, or a tensor of its own); gate_sigmoid: the gate's activation is the logistic function, not silu.
-// a_ch (or null): 32-bit pre-activations of a decay per key channel, [n_tokens, a_stride] with H * dk columns; then
-// dt_bias has H * dk entries.
 // (delta_chunks.hip) Returns 1, with nothing launched, for sizes and alignments that the chunks do not take.
 int tl_delta_chunks(const void* qkv, int stride, const void* proj, int proj_stride, int b_off, int a_off, const float* A_log, const float* dt_bias,
                     float* state, long long state_stride, const int32_t* qo_indptr, const int32_t* slot_ids, float* o_raw, int t_first, int t_last,
@@ -1324,6 +1319,11 @@ int tl_memory_chunks(const void* proj, int stride, int q_off, int k_off, int v_o
                      float cap, float* state, long long state_stride, const int32_t* qo_indptr, const int32_t* slot_ids, float* o_raw, float* den,
                      int t_first, int t_last, int rows, int H, int dk, int dv, float* ws, long long floats, hipStream_t stream);
 
+// qkv, proj, out as the kernels describe; state: S^T of head h at state + slot * state_stride + h * dv * dk;
+// o_raw: workspace of n_tokens * H * dv floats.  gate: the matrix whose H * dv columns from gate_off hold the output
+// gate (proj itself, or a tensor of its own); gate_sigmoid: the gate's activation is the logistic function, not silu.
+// a_ch (or null): 32-bit pre-activations of a decay per key channel, [n_tokens, a_stride] with H * dk columns; then
+// dt_bias has H * dk entries.
 // ws (ws_floats of tl_chunk_floats): a bfloat16 step's first single_rows rows, one token each, take the kernel for such
 // rows, the others go by chunks of tokens on the matrix cores, if sizes and alignments allow it.
 TL_EXPORT int tl_gated_delta(const void* qkv, int qkv_stride, const void* proj, int proj_stride, int gate_off, int b_off,
