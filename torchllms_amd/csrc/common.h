@@ -50,6 +50,21 @@ __device__ __forceinline__ float limited_gate(float gate, float up, float limit,
   return g / (1.0f + expf(-slope * g)) * (u + 1.0f);
 }
 
+// 64 lanes x 16 bytes from `src` (per lane) to LDS at byte offset `lds_at` (wave-uniform) + 16 * lane.
+// Written as assembly, not as the compiler's builtin: the compiler knows that the builtin writes LDS
+// and, unable to tell the buffers apart, waits for every outstanding load before the first LDS read
+// that follows, which would leave no load in flight during the multiplication.  A kernel that uses it
+// counts its loads itself (s_waitcnt vmcnt) and has no other vector memory loads meanwhile.
+__device__ __forceinline__ void load_to_lds(const void* src, uint32_t lds_at) {
+  asm volatile(
+      "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %0, off"
+      :
+      : "v"(src), "s"(lds_at)
+      : "m0", "memory");
+}
+
 // Sum over the 64 lanes of a wave in a fixed butterfly order; every lane gets the result.
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

@@ -34,18 +34,6 @@ typedef float float4_e __attribute__((ext_vector_type(4)));
 constexpr int kStepE = 64;    // k per step: 8 pieces of 16 bytes a row
 constexpr int kXcds = 8;
 
-// 64 lanes x 16 bytes from `src` (per lane) to LDS at byte offset `lds_at` (wave-uniform) + 16 * lane; assembly because the
-// kernel counts its loads itself (see gemm_wide.hip).
-__device__ __forceinline__ void rows_to_lds(const bf16_t* src, uint32_t lds_at) {
-  asm volatile(
-      "s_mov_b32 m0, %1\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, off"
-      :
-      : "v"(src), "s"(lds_at)
-      : "m0", "memory");
-}
-
 // silu(gate) * up of four columns.  rounded: the two products and the activation are rounded to bfloat16 on the way, as dense
 // layers' are (silu_mul of a product stored in bfloat16); otherwise the result alone is.
 __device__ __forceinline__ bf16x4_e gated(const float4_e& gate, const float4_e& up, bool rounded) {
@@ -151,9 +139,9 @@ expert_tile_kernel(const bf16_t* __restrict__ rows, const bf16_t* __restrict__ w
   const uint32_t w_at = __builtin_amdgcn_readfirstlane(base + (BM + wave * S::kWLoads * 8) * kStepE * 2);
   auto issue = [&](int step, int buffer) {
 #pragma unroll
-    for (int i = 0; i < S::kALoads; ++i) rows_to_lds(asrc[i] + step * kStepE, a_at + (buffer * S::kStage + i * 8 * kStepE) * 2);
+    for (int i = 0; i < S::kALoads; ++i) load_to_lds(asrc[i] + step * kStepE, a_at + (buffer * S::kStage + i * 8 * kStepE) * 2);
 #pragma unroll
-    for (int i = 0; i < S::kWLoads; ++i) rows_to_lds(wsrc[i] + step * kStepE, w_at + (buffer * S::kStage + i * 8 * kStepE) * 2);
+    for (int i = 0; i < S::kWLoads; ++i) load_to_lds(wsrc[i] + step * kStepE, w_at + (buffer * S::kStage + i * 8 * kStepE) * 2);
   };
 
   float4_e acc[NT][MT];
@@ -292,9 +280,9 @@ expert_wide_tile_kernel(const bf16_t* __restrict__ rows, const bf16_t* __restric
   const uint32_t w_at = __builtin_amdgcn_readfirstlane(base + kWideM * kWideStep * 2 + wave * 4 * 1024);
   auto issue = [&](int step, int buffer) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) rows_to_lds(src[j] + step * kWideStep, a_at + buffer * kWideStage * 2 + j * 1024);
+    for (int j = 0; j < 2; ++j) load_to_lds(src[j] + step * kWideStep, a_at + buffer * kWideStage * 2 + j * 1024);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) rows_to_lds(src[2 + j] + step * kWideStep, w_at + buffer * kWideStage * 2 + j * 1024);
+    for (int j = 0; j < 4; ++j) load_to_lds(src[2 + j] + step * kWideStep, w_at + buffer * kWideStage * 2 + j * 1024);
   };
   float4_e acc[NT][MT];
 #pragma unroll

@@ -29,18 +29,6 @@ constexpr int BK = 16;  // products that are added among themselves before they 
 // tiles of plain fused multiply-adds before, 95 + 73 + 388 + 266 now; 2,048 rows of the 8B shape's gate/up: 4.0 ms, 120 TFLOP/s.
 __device__ __attribute__((aligned(16))) const float kZeroPiece[4] = {0.f, 0.f, 0.f, 0.f};
 
-// 64 lanes x 16 bytes from `src` (per lane) to LDS at byte offset `lds_at` (wave-uniform) + 16 * lane.  Assembly for the
-// reason gemm_wide.hip gives: the kernel counts its loads itself.
-__device__ __forceinline__ void piece_to_lds(const float* src, uint32_t lds_at) {
-  asm volatile(
-      "s_mov_b32 m0, %1\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, off"
-      :
-      : "v"(src), "s"(lds_at)
-      : "m0", "memory");
-}
-
 template <int BM, int BN, int WM, int WN, int kStepF, int kStages, bool kVec>
 __global__ void __launch_bounds__(256, 2)  // (two waves a SIMD: with 256 registers the compiler keeps sums out of the accumulation registers)
 gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw, float* __restrict__ C, int ldc, int M,
@@ -85,7 +73,7 @@ gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __restri
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
       const int k = step * kStepF + piece[j];
-      piece_to_lds(k < K ? src[j] + k : kZeroPiece, at0 + buffer * kStage * (int)sizeof(float) + j * 1024);
+      load_to_lds(k < K ? src[j] + k : kZeroPiece, at0 + buffer * kStage * (int)sizeof(float) + j * 1024);
     }
   };
   // -- other rows: a thread moves pieces tid, tid + 256, ... of the buffer

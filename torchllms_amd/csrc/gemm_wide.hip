@@ -35,21 +35,6 @@ constexpr int kStepK = 128;            // k per step: 16 pieces of 8 elements
 constexpr int kRowElems = kStepK;      // an LDS row holds one step of one row
 constexpr int kStripElems = 16 * kRowElems;
 
-// 64 lanes x 16 bytes from `src` (per lane) to LDS at byte offset `lds_at` (wave-uniform) + 16 * lane.
-// Written as assembly, not as the compiler's builtin: the compiler knows that the builtin writes LDS
-// and, unable to tell the buffers apart, waits for every outstanding load before the first LDS read
-// that follows, which would leave no load in flight during the multiplication.  The kernel counts
-// its loads itself (s_waitcnt vmcnt) and has no other vector memory loads.
-__device__ __forceinline__ void load_to_lds(const bf16_t* src, uint32_t lds_at) {
-  asm volatile(
-      "s_mov_b32 m0, %1\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, off"
-      :
-      : "v"(src), "s"(lds_at)
-      : "m0", "memory");
-}
-
 // MC: chunks of 16 rows of A (M <= 16 MC).  NCW: strips of 16 columns per wave.
 // STAGES: buffers; the loads of STAGES - 1 steps are in flight while one step is multiplied.
 template <int MC, int NCW, int STAGES>
