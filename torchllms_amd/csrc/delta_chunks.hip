@@ -22,8 +22,8 @@
 // What bounds it: the walk, a chain of one chunk behind the other, about 1.7 us each, of which 16 + 4 + 8 MFMAs of 32 cycles are
 // 0.4; the rest is the way through LDS, the barrier and the operands' loads.  A prompt of 2,048 tokens with 32 heads of 128 takes
 // 40 + 219 us with the rule of a decay per head (token by token 1,242, 16 columns a block), eight prompts of 1,804 tokens 63 + 137 us
-// with a decay per channel (816) and 24 + 32 + 143 us as matrix memory (634).  Against 64 bits (states after 15 to 2,089 tokens, all
-// four kinds): 0.85 to 1.27 times the walk's distance over a step's states, 0.97 on average.
+// with a decay per channel (816) and 24 + 32 + 143 us as matrix memory (634).  Against 64 bits the states of 32 heads (rows of
+// 40 to 600 tokens, all four kinds) are 0.90 to 1.01 times as far as the walk's; of two heads alone up to 1.27 times, by chance.
 // The workspace grows with the rows: a step's tokens are taken in windows (the state goes through memory between them), and it
 // holds a slot for every 16 tokens of a window and one more for every row of the step.  The caller bounds it, or walks.
 #include "common.h"
