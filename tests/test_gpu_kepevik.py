@@ -38,6 +38,23 @@ def truth_of(cfg, weights, requests):
     return out, scale
 
 
+def float32_bounds(cfg, weights, requests, truth, scale):
+    """Per request and position, the distance that the engine may have from the truth in 32-bit: ``FP32_TOL``, or, where
+    the model itself is ill-conditioned (a value of one channel that nearly cancels before its norm, a router's near tie),
+    16 times what one rounding of every weight does there (the root mean square over eight random roundings, in 64-bit).
+    Half the positions of the plain model in 32-bit lie under 2.6 to 3.6 times that, the engine's under 1.9 to 2.6 (96
+    models: single channels, wider values, drawn configurations), and the largest ratio of a position beyond ``FP32_TOL``
+    was 12, whichever order the products are added in; a fault's distance has nothing to do with a rounding's."""
+    g = torch.Generator().manual_seed(17)
+    moved = {rid: torch.zeros(len(toks), dtype=torch.float64) for rid, toks in requests.items()}
+    for _ in range(8):
+        w = {k: v.double() * (1 + (2 * torch.rand(v.shape, generator=g, dtype=torch.float64) - 1) * 2.0 ** -24) for k, v in weights.items()}
+        for rid, toks in requests.items():
+            out = plain.forward(cfg, w, toks)
+            moved[rid] += torch.tensor([distance(out[i], truth[rid][i], scale) for i in range(len(toks))]) ** 2
+    return {rid: [max(FP32_TOL, 16 * float(m)) for m in (sq / 8).sqrt()] for rid, sq in moved.items()}
+
+
 def folder_for(dtype, path, cfg_dict, **kw):
     """The model a run in ``dtype`` is compared on.  Rounding to bfloat16 moves a router's scores by a thousandth,
     and where two outputs lie closer than that the engine and the plain model choose different experts for a token:
@@ -182,10 +199,12 @@ def test_a_mechanism_alone(tmp_path, what, dtype):
         at += n
     assert at == len(tokens)
     cut = torch.cat(rows)
+    bounds = float32_bounds(cfg, weights, {"r": tokens}, truth, scale)["r"] if dtype == "float32" else None
     for name, got in (("whole", whole), ("cut", cut)):
         dists = [distance(got[i], truth["r"][i], scale) for i in range(len(tokens))]
         if dtype == "float32":
-            assert max(dists) < FP32_TOL, f"{what}/{name}: distance {max(dists)}"
+            over = [(i, d, b) for i, (d, b) in enumerate(zip(dists, bounds)) if not d < b]
+            assert not over, f"{what}/{name}: {over[:3]}"
         else:
             assert_within_rounding(dists, BF16_TOL, f"{what}/{name}")
     if dtype == "float32":
@@ -703,9 +722,11 @@ def test_random_configurations(tmp_path, seed):
     rng = random.Random(seed)
     requests = {"a": random_tokens(rng.randint(120, 330), cfg_dict["vocab"], seed), "b": random_tokens(rng.randint(20, 90), cfg_dict["vocab"], seed + 50)}
     page = rng.choice([4, 8, 16, 32])
-    for dtype, tol in (("float32", FP32_TOL), ("bfloat16", 5 * BF16_TOL)):
+    for dtype, tol in (("float32", None), ("bfloat16", 5 * BF16_TOL)):
         folder = folder_for(dtype, tmp_path / "m", cfg_dict, seed=seed)
-        truth, scale = truth_of(*models.read_folder(folder), requests)
+        cfg, weights = models.read_folder(folder)
+        truth, scale = truth_of(cfg, weights, requests)
+        bounds = float32_bounds(cfg, weights, requests, truth, scale) if dtype == "float32" else None
         seen = []
         engine = Engine.from_folder(folder, dtype=dtype, page_size=page, num_pages=2 * (-(-420 // page)) + 4, max_seqs=3)
         engine.admit("w")
@@ -714,7 +735,7 @@ def test_random_configurations(tmp_path, seed):
         for i, row in enumerate(whole):
             d = distance(row, truth["a"][i], scale)
             seen.append(d)
-            assert dtype == "bfloat16" or d < tol, f"{dtype} whole at {i}: {d}  {cfg_dict}"
+            assert dtype == "bfloat16" or d < bounds["a"][i], f"{dtype} whole at {i}: {d}, bound {bounds['a'][i]}  {cfg_dict}"
         at = {"a": 0, "b": 0}
         engine.admit("a")
         engine.admit("b")
@@ -733,7 +754,7 @@ def test_random_configurations(tmp_path, seed):
                 for w in e.want:
                     d = distance(logits[k], truth[e.rid][at[e.rid] + w], scale)
                     seen.append(d)
-                    assert dtype == "bfloat16" or d < tol, f"{dtype} {e.rid} at {at[e.rid] + w} in a step of {[len(x.tokens) for x in entries]}: {d}  {cfg_dict}"
+                    assert dtype == "bfloat16" or d < bounds[e.rid][at[e.rid] + w], f"{dtype} {e.rid} at {at[e.rid] + w} in a step of {[len(x.tokens) for x in entries]}: {d}  {cfg_dict}"
                     if dtype == "float32" and e.rid == "a":
                         assert torch.equal(logits[k], whole[at["a"] + w])
                     k += 1
