@@ -61,6 +61,8 @@ def test_engines_built_from_one_table_agree_bit_for_bit(tmp_path, monkeypatch):
     assert third.kernel_table() == library
     x = torch.zeros((4, 256), dtype=torch.bfloat16, device="cuda:0")
     assert ops.linear_choice(x, third.model.blocks[0].mixer.wo, "sum") is None
+    many = torch.zeros((24, 256), dtype=torch.bfloat16, device="cuda:0")  # rows of which the rule has a kernel of its own
+    assert ops.linear_choice(many, third.model.blocks[0].mixer.wqkv, "qkv") is None
     near = run_trace(third, steps)
     worst = max((near[k] - want[k]).abs().max().item() for k in want)
     assert worst < 0.5  # the same model through other kernels: near, not equal

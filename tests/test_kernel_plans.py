@@ -114,13 +114,14 @@ def test_the_tuned_table_decides_per_shape_rows_and_use():
 
 
 def test_which_candidates_are_charged_a_kernel_of_their_own_for_the_second_half():
-    stream, whole, split = ("stream", 4), ("wide", 2, 1, 3), ("wide", 1, 4, 3)
-    for choice in (None, stream, whole, split):
+    stream, whole, split, narrow = ("stream", 4), ("wide", 2, 1, 3), ("wide", 1, 4, 3), ("narrow",)
+    for choice in (None, stream, whole, split, narrow):
         assert products.fuses_tail(choice, "plain")
     # the streaming product adds itself to the residual rows and leaves the norm's statistics; the library cannot
     assert [products.fuses_tail(c, "sum") for c in (None, stream, whole, split)] == [False, True, True, True]
     assert [products.fuses_tail(c, "glu") for c in (None, stream, whole, split)] == [False, True, True, False]
     assert [products.fuses_tail(c, "qkv") for c in (None, stream, whole, split)] == [False, True, False, True]
+    assert [products.fuses_tail(narrow, use) for use in ("plain", "glu", "qkv", "sum")] == [True, False, True, True]
 
 
 @pytest.mark.parametrize("n, k, narrow", [(3072, 2048, True), (4096, 2048, True), (96, 128, True), (4112, 1024, True), (2048, 8192, False),
@@ -131,6 +132,34 @@ def test_which_products_of_17_to_32_rows_run_by_the_kernel_for_few_columns(n, k,
         for use in ops.LINEAR_USES:
             assert (ops.linear_choice(x[:m], w, use) == ("narrow",)) == (narrow and use in ("plain", "qkv"))
     assert ops.linear_choice(x[:16], w) != ("narrow",) and ops.linear_choice(x, w) != ("narrow",)
+
+
+def test_the_table_decides_before_the_rule_of_sizes():
+    """Also for 17 to 32 rows of a shape that the rule gives to the kernel for few columns; and where the table has a use
+    of the same shape only as a sum, a model that asks for the plain product gets that launch, at every row count."""
+    w, x = torch.empty((3072, 2048), dtype=torch.bfloat16), torch.empty((24, 2048), dtype=torch.bfloat16)
+    saved = dict(products.LINEAR_CHOICE)
+    try:
+        products.LINEAR_CHOICE.clear()
+        ops.load_kernel_table({"3072,2048,32,plain": None, "3072,2048,32,qkv": ["wide", 1, 4, 3]})
+        assert ops.linear_choice(x, w) is None and ops.linear_choice(x, w, "qkv") == ("wide", 1, 4, 3)
+        ops.load_kernel_table({"3072,2048,32,plain": ["narrow"], "4096,4096,32,qkv": ["narrow"]})
+        assert ops.linear_choice(x, w) == ("narrow",) and ops.kernel_table()["4096,4096,32,qkv"] == ["narrow"]
+        for bad in ({"256,256,64,plain": ["narrow"]}, {"256,256,16,plain": ["narrow"]}, {"256,200,32,plain": ["narrow"]},
+                    {"256,256,32,glu": ["narrow"]}, {"256,256,32,sum": ["narrow"]}, {"256,256,32,plain": ["narrow", 4]}):
+            with pytest.raises(ValueError, match="kernel table"):
+                ops.load_kernel_table(bad)
+        ops.clear_kernel_table()
+        old = {"3072,2048,8,sum": ["stream", 4], "3072,2048,32,sum": ["wide", 1, 8, 3], "3072,2048,64,sum": None}
+        ops.load_kernel_table(old, [((3072, 2048), "sum")])
+        assert len(ops.kernel_table()) == 3
+        ops.load_kernel_table(old, [((3072, 2048), "plain")])
+        assert ops.linear_choice(x, w) == ("wide", 1, 8, 3) and ops.linear_choice(x[:8], w) == ("stream", 4)
+        ops.load_kernel_table(dict(old, **{"3072,2048,32,plain": None}), [((3072, 2048), "plain")])
+        assert ops.linear_choice(x, w) is None
+    finally:
+        products.LINEAR_CHOICE.clear()
+        products.LINEAR_CHOICE.update(saved)
 
 
 def test_which_launches_of_the_wide_kernel_fit_lds():

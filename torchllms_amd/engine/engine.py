@@ -124,7 +124,7 @@ class Engine:
         from ..kernels import ops
 
         if kernel_table is not None:
-            ops.load_kernel_table(kernel_table)
+            ops.load_kernel_table(kernel_table, [(shape, use) for shape, use, _ in self.model.linear_weights()])
         if dtype == torch.bfloat16 and tune_kernels:
             # which matrix-product kernel serves decode steps best is measured, not guessed; before
             # the pool is sized, so that what the measurement borrows is free again for pages

@@ -234,10 +234,17 @@ def gemm_wide(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype = torch.b
 
 
 NARROW_MAX_ROWS = 32
-#: the most elements of a row of x that a CU may have to take in, ``k * ceil(n / 4096)`` (256 CUs, blocks of 16 columns): up
-#: to here the kernel for few columns is the faster one, 5.3 to 8.0 us for 7.6 to 9.7, beyond it 12.4 for 11.8 (4,096 x 4,096)
+#: the most elements of a row of x that a CU may have to take in, k for every round of blocks of 16 columns on all CUs (4,096
+#: columns on 256): up to here the kernel for few columns is the faster one, 5.3 to 8.0 us for 7.6 to 9.7, beyond it 12.4 for
+#: 11.8 (4,096 x 4,096)
 NARROW_MAX_ELEMENTS = 2048
-NARROW_MAX_ROUNDS = 2  # of 4,096 columns: many short blocks lose again (8,192 x 1,024 7.9 for 8.8, 16,384 x 512 8.5 for 7.1)
+NARROW_MAX_ROUNDS = 2  # many short blocks lose again (8,192 x 1,024 7.9 for 8.8, 16,384 x 512 8.5 for 7.1)
+
+
+def narrow_by_size(n: int, k: int) -> bool:
+    """Whether the kernel for few columns serves a shape of 17 to 32 rows that was never measured."""
+    rounds = -(-n // (16 * device_facts()[0]))
+    return rounds <= NARROW_MAX_ROUNDS and k * rounds <= NARROW_MAX_ELEMENTS
 
 
 def gemm_narrow(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
@@ -465,6 +472,7 @@ def wide_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
 #:   ("stream", waves[, cols])                     the weight-streaming kernel (waves 0 = its own rule;
 #:                                                 cols: columns per block of the gated form, 8 or 16)
 #:   ("wide", strips_per_wave, k_splits, stages)   the kernel whose blocks share the activations
+#:   ("narrow",)                                   the kernel for few columns (17 to 32 rows, uses of ``NARROW_USES``)
 #:   None                                          the library
 #: Shapes never measured follow the size rule of ``linear_choice``.
 LINEAR_CHOICE: dict = {}
@@ -486,6 +494,7 @@ def wide_fits(rows: int, strips_per_wave: int, stages: int) -> bool:
 #: ``linear_to_sum``) as a term of the residual sum, where the norm that follows adds up a split
 #: product for nothing
 LINEAR_USES = ("plain", "glu", "qkv", "sum")
+NARROW_USES = ("plain", "qkv")  # (a gate and a sum are taken by other kernels into themselves for less)
 #: microseconds that a small kernel between large ones costs in a replayed decode step (measured as
 #: the difference between graphs with and without it: 2.7 to 3.1 for a norm of 1 to 64 rows; a kernel
 #: trace shows 4.6 and more for every dispatch, an empty one included, which is the profiler's own);
@@ -512,16 +521,17 @@ def fuses_tail(choice, use: str) -> bool:
         return False
     if choice[0] == "stream" or use == "sum":
         return True
+    if choice[0] == "narrow":
+        return use == "qkv"
     return choice[2] == 1 if use == "glu" else choice[2] > 1  # the gate ends a whole product, the rotation a split one
 
 
 def linear_choice(x: torch.Tensor, w: torch.Tensor, use: str = "plain"):
     """Which bfloat16 kernel runs ``x @ w.T``: a tuple as in the table above, or None for the library.
-    17 to 32 rows of small matrices run by the kernel for few columns (``NARROW_MAX_ELEMENTS``), except those whose gate or
-    sum another kernel takes into itself for less.  For the rest
-    what the table holds decides.  A shape it does not hold follows a fixed rule: up to 16 rows the
+    What the table holds decides.  A shape it does not hold follows a fixed rule: up to 16 rows the
     weight-streaming kernel (its own choice of waves) for matrices of at most ``STREAM_MAX_ELEMENTS``
-    elements, the library otherwise."""
+    elements, 17 to 32 rows of small matrices the kernel for few columns (``narrow_by_size``), except for uses that it
+    does not take, the library otherwise."""
     m = x.shape[0]
     if m <= STREAM_MAX_ROWS:
         if not stream_supported(x, w):
@@ -532,10 +542,10 @@ def linear_choice(x: torch.Tensor, w: torch.Tensor, use: str = "plain"):
         return ("stream", 0) if w.shape[0] * w.shape[1] <= STREAM_MAX_ELEMENTS else None
     if not wide_supported(x, w):
         return None
-    rounds = -(-w.shape[0] // 4096)
-    if use in ("plain", "qkv") and m <= NARROW_MAX_ROWS and rounds <= NARROW_MAX_ROUNDS and w.shape[1] * rounds <= NARROW_MAX_ELEMENTS:
-        return ("narrow",)
-    return LINEAR_CHOICE.get((w.shape[0], w.shape[1], row_bucket(m), use))
+    key = (w.shape[0], w.shape[1], row_bucket(m), use)
+    if key in LINEAR_CHOICE:
+        return LINEAR_CHOICE[key]
+    return ("narrow",) if use in NARROW_USES and m <= NARROW_MAX_ROWS and narrow_by_size(*w.shape) else None
 
 
 # ----------------------------------------------------------------------------- the table, outside the process
@@ -550,11 +560,15 @@ def kernel_table(shapes=None) -> dict:
     return out
 
 
-def load_kernel_table(table) -> None:
+def load_kernel_table(table, shapes=None) -> None:
     """Put the entries of ``table`` (a dict as ``kernel_table`` returns, or the path of a JSON file
     holding one) into the table; they replace what was measured for the same keys, and
     ``tune_linear`` leaves them alone.  Every entry is checked: a table from somewhere else must not
-    be able to ask a kernel for a launch it does not have."""
+    be able to ask a kernel for a launch it does not have.
+
+    ``shapes``: the ``((n, k), use)`` pairs that a model will ask for.  Where it asks for a "plain" product of which the table
+    knows only the "sum", that entry serves both: layers that make a tensor of a branch's result at once used to ask for
+    its last product as a sum, and tables saved then hold nothing else for it."""
     import json
     import os
 
@@ -575,11 +589,16 @@ def load_kernel_table(table) -> None:
             ok = False
             if choice and choice[0] == "stream" and bucket <= STREAM_MAX_ROWS:
                 ok = len(choice) in (2, 3) and choice[1] in STREAM_WAVE_CHOICES and (len(choice) == 2 or (use == "glu" and choice[2] in (8, 16)))
+            elif choice and choice[0] == "narrow":
+                ok = len(choice) == 1 and STREAM_MAX_ROWS < bucket <= NARROW_MAX_ROWS and use in NARROW_USES and k % 128 == 0
             elif choice and choice[0] == "wide" and bucket > STREAM_MAX_ROWS:
                 ok = len(choice) == 4 and choice[1:] in WIDE_CHOICES and k % 128 == 0 and choice[2] <= k // 128 and wide_fits(bucket, choice[1], choice[3])
             if not ok:
                 raise ValueError(f"kernel table: entry {key!r} -> {list(choice)!r} names no launch of a kernel here")
         entries[(n, k, bucket, use)] = choice
+    for (n, k), use in shapes or ():
+        if use == "plain" and not any((n, k, bucket, "plain") in entries for bucket in ROW_BUCKETS):
+            entries.update({(n, k, bucket, "plain"): entries[(n, k, bucket, "sum")] for bucket in ROW_BUCKETS if (n, k, bucket, "sum") in entries})
     LINEAR_CHOICE.update(entries)
 
 
@@ -690,6 +709,8 @@ def tune_linear(weights, out_dtype: torch.dtype = torch.bfloat16, use: str = "pl
             candidates = [("wide",) + c for c in WIDE_CHOICES if c[1] <= k // 128 and wide_fits(bucket, c[0], c[2])]
             # (two buffers are only tried where three do not fit)
             candidates = [c for c in candidates if c[3] == 3 or not wide_fits(bucket, c[1], 3)]
+            if bucket <= NARROW_MAX_ROWS and use in NARROW_USES:
+                candidates.insert(0, ("narrow",))
         else:
             candidates = []
         timed += [(choice, cost(bucket, choice, run(choice))) for choice in candidates]
