@@ -58,15 +58,12 @@ __device__ __forceinline__ void qkv_finish(const float* sums, int row, int n, co
     for (int pi = 0; pi < 2; ++pi) {
       if (d + 2 * pi < qa.rotary_dim) {
         const float2 cs = o.cs[pi];
-        const float x0 = x[2 * pi], x1 = x[2 * pi + 1];
-        if constexpr (sizeof(T) == sizeof(float)) {
-          const float2 r = rotated(x0, x1, cs);  // (bit for bit the rotary kernel's)
-          x[2 * pi] = r.x;
-          x[2 * pi + 1] = r.y;
-        } else {
-          x[2 * pi] = x0 * cs.x - x1 * cs.y;
-          x[2 * pi + 1] = x1 * cs.x + x0 * cs.y;
-        }
+        float2 r = rotated(x[2 * pi], x[2 * pi + 1], cs);  // (float: bit for bit the rotary kernel's)
+        // (the bfloat16 products round the second sum's other product alone: a float's last bit, which the sums' own order
+        // moves far oftener; written out, so that all of them give the same bits)
+        if constexpr (sizeof(T) < sizeof(float)) r.y = __builtin_fmaf(x[2 * pi + 1], cs.x, x[2 * pi] * cs.y);
+        x[2 * pi] = r.x;
+        x[2 * pi + 1] = r.y;
       }
     }
   }
