@@ -283,7 +283,7 @@ def test_matrix_core_attention_with_a_table_of_distances(Hq, Hk, d, dv, page, wi
     want = ops.attention_generic(q, Hq, Hk, d, kp, vp, seq, pos, bt, window, scale, v_head_dim=dv, **kw).float()
     flat = ops.attention_generic(q, Hq, Hk, d, kp, vp, seq, pos, bt, window, scale, v_head_dim=dv).float()
     assert window == 1 or (want - flat).abs().max() > 0.3  # (the table does decide)
-    for split in (None, 64, 128):
+    for split in (None, 64, 128, 1024):  # (1,024: left whole, by eight waves a block)
         got = torch.zeros((len(positions), Hq * dv), dtype=torch.bfloat16, device=DEV)
         for at in range(0, dv, d):
             ops.attention_decode(q, Hq, Hk, d, kp, vp, seq, pos, bt, window, scale, min(max(positions) + 1, window + 15) if window else max(positions) + 1,
@@ -335,7 +335,7 @@ def test_groups_of_query_heads_over_one_head_of_the_pages(H, per, d, page):
     want = torch.stack([_plain_attention(q[i].float(), rows, rows, p, 0, 0, scale, 0.0, None, sinks, H) for i, p in enumerate(ps)])
     no_sink = torch.stack([_plain_attention(q[i].float(), rows, rows, p, 0, 0, scale, 0.0, None, None, H) for i, p in enumerate(ps)])
     assert (want - no_sink).abs().max() > 0.3
-    for split in (None, 64):
+    for split in (None, 64, 1024):  # (1,024: left whole, by eight waves where a group's outputs are small)
         got = ops.attention_decode(q.view(len(ps), H * d).to(DEV), H, H // per, d, kp, kp, torch.zeros(len(ps), dtype=torch.int32, device=DEV),
                                    torch.tensor(ps, dtype=torch.int32, device=DEV), bt, 0, scale, 500, split_size=split, **kw)
         assert (got.float().cpu().view(len(ps), H, d).double() - want).abs().max() < 3e-2 * float(want.abs().max())

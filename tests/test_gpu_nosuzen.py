@@ -317,7 +317,7 @@ def test_matrix_core_attention_with_kept_first_keys_and_wide_values(Hq, Hk, Hv, 
     pos = torch.tensor(positions, dtype=torch.int32, device=DEV)
     seq = torch.zeros(len(positions), dtype=torch.int32, device=DEV)
     want = ops.attention_generic(q, Hq, Hk, d, kp, vp, seq, pos, bt, window, scale, v_head_dim=dv, **kw).float()
-    for split in (None, 64, 128):
+    for split in (None, 64, 128, 1024):  # (1,024: left whole, by eight waves a block)
         got = torch.zeros((len(positions), Hq * dv), dtype=torch.bfloat16, device=DEV)
         for at in range(0, dv, d):
             ops.attention_decode(q, Hq, Hk, d, kp, vp, seq, pos, bt, window, scale, min(max(positions) + 1, window + 15), out=got,

@@ -310,7 +310,7 @@ def test_matrix_core_attention_with_a_bias_by_distance(Hq, Hk, d, dv, page, wind
     want = ops.attention_generic(q, Hq, Hk, d, kp, vp, seq, pos, bt, window, scale, v_head_dim=dv, **kw).float()
     flat = ops.attention_generic(q, Hq, Hk, d, kp, vp, seq, pos, bt, window, scale, v_head_dim=dv, softcap=cap).float()
     assert window == 1 or (want - flat).abs().max() > 0.3  # (the bias does decide)
-    for split in (None, 64, 128):
+    for split in (None, 64, 128, 1024):  # (1,024: left whole, by eight waves a block)
         got = torch.zeros((len(positions), Hq * dv), dtype=torch.bfloat16, device=DEV)
         for at in range(0, dv, d):
             ops.attention_decode(q, Hq, Hk, d, kp, vp, seq, pos, bt, window, scale, min(max(positions) + 1, window + 15), out=got,

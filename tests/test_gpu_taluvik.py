@@ -624,6 +624,10 @@ def test_matrix_core_attention_agrees_with_the_plain_kernel(head_dim):
     plain_out = ops.attention_generic(qkv, H, G, head_dim, k_pages, v_pages, ctx.token_seq, ctx.positions, ctx.block_tables[0],
                                       0, scale, v_head_dim=head_dim, **extras).float()
     assert (fast - plain_out).abs().max() < 0.03, (fast - plain_out).abs().max()
+    for split in (64, 1024):  # the single tokens in splits, and left whole by eight waves a block
+        single = ops.attention_decode(qkv[:2], H, G, head_dim, k_pages, v_pages, ctx.token_seq[:2], ctx.positions[:2], ctx.block_tables[0],
+                                      0, scale, 201, split_size=split, **extras).float()
+        assert (single - plain_out[:2]).abs().max() < 0.03, (split, (single - plain_out[:2]).abs().max())
     # what the comparison would miss if both forgot the same thing: the plain kernel alone notices each of the three
     for change in (dict(extras, softcap=0.0), dict(extras, chunk=0), dict(extras, sinks=None)):
         other = ops.attention_generic(qkv, H, G, head_dim, k_pages, v_pages, ctx.token_seq, ctx.positions, ctx.block_tables[0],
