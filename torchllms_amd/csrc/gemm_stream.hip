@@ -431,8 +431,6 @@ int launch(const bf16_t* A, int lda, const bf16_t* W, int ldw, void* C, int ldc,
   if constexpr (MR == 1) {  // (a pair is one row)
     if (na.w_select != nullptr) {
       if (epi == kGated) return launch_typed<MR, WAVES, bf16_t, kGated, true>(A, lda, W, ldw, (bf16_t*)C, ldc, M, N, K, qa, na, pairs, stream);
-      if (epi == kGatedHalf) return launch_typed<MR, WAVES, bf16_t, kGatedHalf, true>(A, lda, W, ldw, (bf16_t*)C, ldc, M, N, K, qa, na, pairs, stream);
-      if (out_dtype == TL_BF16) return launch_typed<MR, WAVES, bf16_t, kPlain, true>(A, lda, W, ldw, (bf16_t*)C, ldc, M, N, K, qa, na, pairs, stream);
       return launch_typed<MR, WAVES, float, kPlain, true>(A, lda, W, ldw, (float*)C, ldc, M, N, K, qa, na, pairs, stream);
     }
   }
@@ -544,18 +542,18 @@ static int run_pairs(const char* who, const void* A, int lda, const void* W, int
   return run(A, lda, W, ldw, C, ldc, pairs > 0 ? 1 : 0, N, K, out_dtype, waves, epi, QkvArgs{}, na, stream, pairs);
 }
 
+// C [pairs, N] 32-bit.
 TL_EXPORT int tl_gemm_stream_select(const void* A, int lda, const void* W, int ldw, void* C, int ldc, int pairs, int row_share, int N, int K,
-                                    int out_dtype, int waves, const int32_t* w_select, long long w_stride, int w_count,
+                                    int waves, const int32_t* w_select, long long w_stride, int w_count,
                                     hipStream_t stream) {
-  return run_pairs("gemm_stream_select", A, lda, W, ldw, C, ldc, pairs, row_share, N, K, out_dtype, waves, kPlain, w_select, w_stride, w_count, stream);
+  return run_pairs("gemm_stream_select", A, lda, W, ldw, C, ldc, pairs, row_share, N, K, TL_F32, waves, kPlain, w_select, w_stride, w_count, stream);
 }
 
+// C [pairs, N] bfloat16.
 TL_EXPORT int tl_gemm_stream_glu_select(const void* A, int lda, const void* W, int ldw, void* C, int ldc, int pairs, int row_share, int N, int K,
-                                        int waves, int cols, const int32_t* w_select, long long w_stride, int w_count,
+                                        int waves, const int32_t* w_select, long long w_stride, int w_count,
                                         hipStream_t stream) {
-  TL_REQUIRE(cols == 8 || cols == 16, "gemm_stream_glu_select: cols must be 8 or 16");
-  return run_pairs("gemm_stream_glu_select", A, lda, W, ldw, C, ldc, pairs, row_share, N, K, TL_BF16, waves, cols == 8 ? kGatedHalf : kGated,
-                   w_select, w_stride, w_count, stream);
+  return run_pairs("gemm_stream_glu_select", A, lda, W, ldw, C, ldc, pairs, row_share, N, K, TL_BF16, waves, kGated, w_select, w_stride, w_count, stream);
 }
 
 // C [M, N] bfloat16 = residual [M, N] + A W^T (the product rounded to bfloat16, then the sum in

@@ -158,9 +158,9 @@ def expert_pair_products(x: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch
         rows, share = torch.empty((pairs, D), dtype=x.dtype, device=x.device), 1
         check(lib.tl_pair_rows(x.data_ptr(), input_weights.data_ptr(), rows.data_ptr(), n, top, D, dtype_code(x.dtype), stream))
     which = ids.data_ptr()
-    check(lib.tl_gemm_stream_glu_select(rows.data_ptr(), D, w_gate_up.data_ptr(), D, mid.data_ptr(), F, pairs, share, F, D, 0, 16, which,
+    check(lib.tl_gemm_stream_glu_select(rows.data_ptr(), D, w_gate_up.data_ptr(), D, mid.data_ptr(), F, pairs, share, F, D, 0, which,
                                         2 * F * D, E, stream))
-    check(lib.tl_gemm_stream_select(mid.data_ptr(), F, w_down.data_ptr(), F, y.data_ptr(), D, pairs, 1, D, F, F32, 0, which, D * F, E, stream))
+    check(lib.tl_gemm_stream_select(mid.data_ptr(), F, w_down.data_ptr(), F, y.data_ptr(), D, pairs, 1, D, F, 0, which, D * F, E, stream))
     return y
 
 
