@@ -534,8 +534,8 @@ def peaks_run(args) -> int:
     """What this GPU reaches at its clocks of today, beside the published figures: a read of 4 GiB by a
     kernel of 16-byte loads, a device-to-device copy (its bytes counted once read, once written), MFMA
     bfloat16 16x16x32 instructions issued from registers alone, the library's product of two
-    8,192 x 8,192 bfloat16 matrices, and plain 32-bit multiply-adds from registers alone (the
-    arithmetic of the 32-bit path's products)."""
+    8,192 x 8,192 bfloat16 matrices, and plain 32-bit multiply-adds from registers alone (on the vector
+    units; the 32-bit path's products take the matrix cores)."""
     import torch
 
     from torchllms_amd.kernels import lib
