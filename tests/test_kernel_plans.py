@@ -134,6 +134,28 @@ def test_which_products_of_17_to_32_rows_run_by_the_kernel_for_few_columns(n, k,
     assert ops.linear_choice(x[:16], w) != ("narrow",) and ops.linear_choice(x, w) != ("narrow",)
 
 
+def test_what_the_kernels_for_17_rows_and_more_do_not_take_stays_with_the_library():
+    """Columns that lie apart, more than two dimensions, matrices without rows or columns: no rule of sizes and no table sends
+    them to a kernel that would refuse them."""
+    bf = torch.bfloat16
+    x, w = torch.empty((24, 256), dtype=bf), torch.empty((96, 256), dtype=bf)
+    refused = [(torch.empty((24, 512), dtype=bf)[:, ::2], w), (x, torch.empty((96, 512), dtype=bf)[:, ::2]),
+               (torch.empty((24, 256, 256), dtype=bf), w), (x, torch.empty((0, 256), dtype=bf)),
+               (torch.empty((24, 0), dtype=bf), torch.empty((96, 0), dtype=bf))]
+    saved = dict(products.LINEAR_CHOICE)
+    try:
+        for table in ({}, {(96, 256, 32, "plain"): ("wide", 1, 2, 3)}):
+            products.LINEAR_CHOICE.clear()
+            products.LINEAR_CHOICE.update(table)
+            assert ops.linear_choice(x, w) is not None
+            for a, b in refused:
+                for use in ops.LINEAR_USES:
+                    assert ops.linear_choice(a, b, use) is None, (a.shape, a.stride(), b.shape, b.stride(), use)
+    finally:
+        products.LINEAR_CHOICE.clear()
+        products.LINEAR_CHOICE.update(saved)
+
+
 def test_the_table_decides_before_the_rule_of_sizes():
     """Also for 17 to 32 rows of a shape that the rule gives to the kernel for few columns; and where the table has a use
     of the same shape only as a sum, a model that asks for the plain product gets that launch, at every row count."""

@@ -463,6 +463,7 @@ def wide_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether the kernel for 17 to 128 rows can take this product at all."""
     return (
         x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and STREAM_MAX_ROWS < x.shape[0] <= WIDE_MAX_ROWS
+        and x.dim() == 2 and w.dim() == 2 and w.shape[0] > 0 and x.shape[1] > 0 and x.stride(1) == 1 and w.stride(1) == 1
         and x.shape[1] % 128 == 0 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
         and w.data_ptr() % 16 == 0
     )
