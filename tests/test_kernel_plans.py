@@ -156,6 +156,14 @@ def test_what_the_kernels_for_17_rows_and_more_do_not_take_stays_with_the_librar
         products.LINEAR_CHOICE.update(saved)
 
 
+def test_float32_products_of_what_is_no_matrix_are_refused_as_kernel_errors():
+    for x in (torch.zeros(4), torch.zeros((2, 3, 4))):
+        with pytest.raises(ops.KernelError):
+            ops.linear_glu(x, torch.zeros((6, 4)))
+        with pytest.raises(ops.KernelError):
+            ops.qkv_rope_store(x, torch.zeros((12, 4)), None, 1, 1, 4, torch.zeros(2, dtype=torch.int32), None, 0, 0, None, None, None, None, 0)
+
+
 def test_the_table_decides_before_the_rule_of_sizes():
     """Also for 17 to 32 rows of a shape that the rule gives to the kernel for few columns; and where the table has a use
     of the same shape only as a sum, a model that asks for the plain product gets that launch, at every row count."""

@@ -47,7 +47,7 @@ def gemm_f32(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = Non
 
 def gemm_f32_few_fits(x: torch.Tensor) -> bool:
     """Whether ``gemm_f32_glu`` and ``gemm_f32_qkv`` take these rows: at most 16, not of extreme length."""
-    return x.dtype == torch.float32 and 0 < x.shape[0] <= 16 and bool(core().tl_gemm_f32_few_fits(x.shape[0], x.shape[1]))
+    return x.dtype == torch.float32 and x.dim() == 2 and 0 < x.shape[0] <= 16 and bool(core().tl_gemm_f32_few_fits(x.shape[0], x.shape[1]))
 
 
 def gemm_f32_glu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
